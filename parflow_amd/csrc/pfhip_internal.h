@@ -24,7 +24,9 @@ struct pfhip_problem {
   double *q2[4];              /* device surface scratch                   */
   double *red_partial;        /* reduction partials (RED_MAX_BLOCKS*8)    */
   double *red_dev;            /* device result slots (PFHIP_RED_SLOTS)    */
-  double *h_red;              /* pinned host result slots (64)            */
+  double *h_red;              /* pinned host result slots, then the
+                                 sequence number of the last results      */
+  unsigned long long red_seq; /* the sequence number last asked for       */
   double *krtab;              /* device kr lookup table, or NULL          */
   double *stat_partial;       /* KINStop partials of the line-search
                                  residual: 2 x stat_nb                    */
