@@ -130,8 +130,7 @@ int  pfhip_nl_function_eval(pfhip_problem *pb, const double *p, double *F,
  *   vy[i + nx*(j + (ny+1)*k)]    nx*(ny+1)*nz
  *   vz[i + nx*(j + ny*k)]        nx*ny*(nz+1)
  * p_old and dt enter only an OverlandKinematic top (q_overlnd / dt);
- * they may be NULL / 0 otherwise.  Overwrites the problem's internal
- * kr*rho buffer. */
+ * they may be NULL / 0 otherwise. */
 int  pfhip_face_velocity(pfhip_problem *pb, const double *p,
                          const double *p_old, double dt, double *vx,
                          double *vy, double *vz, void *stream);
@@ -224,8 +223,7 @@ int  pfhip_vec_inv_test(pfhip_problem *pb, const double *x, double *z,
  * where that term is small.  PL/overlandsum.c:33 (OverlandSum) accumulates
  * only for OverlandFlow patches (type 7), never for OverlandKinematic, so
  * the runoff term here is what the kinematic path has in its place.
- * p_old: the step's initial pressure (overland top only).  Overwrites the
- * problem's internal kr*rho buffer. */
+ * p_old: the step's initial pressure (overland top only). */
 #define PFHIP_WB_TERMS 4
 int  pfhip_water_balance_fluxes(pfhip_problem *pb, const double *p,
                                 const double *p_old, double dt, double *out,

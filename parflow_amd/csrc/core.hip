@@ -378,8 +378,6 @@ extern "C" int pfhip_problem_create(const pfhip_problem_desc *desc,
       if (e != hipSuccess) { pfhip_set_error("hipHostMalloc"); rc = PFHIP_ERR_NOMEM; }
     }
   }
-  if (rc == PFHIP_OK) rc = pfhip_dev_alloc(&pb->krho, ng);
-  if (rc == PFHIP_OK) rc = pfhip_dev_alloc(&pb->dkrho, ng);
   for (int q = 0; q < 4 && rc == PFHIP_OK; q++) rc = pfhip_dev_alloc(&pb->q2[q], pb->n2);
   if (rc == PFHIP_OK) rc = pfhip_dev_alloc(&pb->red_partial, PFHIP_RED_MAX_BLOCKS * PFHIP_MAX_MULTI);
   if (rc == PFHIP_OK) rc = pfhip_dev_alloc(&pb->red_dev, PFHIP_RED_SLOTS);
@@ -394,8 +392,6 @@ extern "C" int pfhip_problem_create(const pfhip_problem_desc *desc,
     if (e != hipSuccess) { pfhip_set_error("hipHostMalloc"); rc = PFHIP_ERR_NOMEM; }
     else memset(pb->h_red, 0, sizeof(double) * (PFHIP_RED_SLOTS + 1));
   }
-  if (rc == PFHIP_OK) rc = pfhip_zero(pb->krho, ng, nullptr);
-  if (rc == PFHIP_OK) rc = pfhip_zero(pb->dkrho, ng, nullptr);
   if (rc == PFHIP_OK && d->vg_table_points > 0) {
     const int N1 = d->vg_table_points + 1;
     double *host = (double *)calloc(7 * (size_t)N1, sizeof(double));
@@ -427,8 +423,6 @@ extern "C" int pfhip_problem_destroy(pfhip_problem *pb)
     if (pb->bcv[f]) hipFree(pb->bcv[f]);
     if (pb->h_bcv[f]) hipHostFree(pb->h_bcv[f]);
   }
-  if (pb->krho) hipFree(pb->krho);
-  if (pb->dkrho) hipFree(pb->dkrho);
   for (int q = 0; q < 4; q++) if (pb->q2[q]) hipFree(pb->q2[q]);
   if (pb->red_partial) hipFree(pb->red_partial);
   if (pb->red_dev) hipFree(pb->red_dev);
@@ -1742,12 +1736,10 @@ static inline Phys phys_of(const pfhip_problem *pb)
   return f;
 }
 
-// out = S (fcn 0) / dS (1) / kr (2) / dkr (3) / kr*rho (4), or both
-// kr*rho and dkr*rho into out, out2 (5); interior cells
+// out = S (what 0) / dS (1) / kr (2) / dkr (3); interior cells
 __global__ __launch_bounds__(256) void k_closure(Geom g, Phys f, int what,
                                                  const double *__restrict__ p,
-                                                 double *__restrict__ out,
-                                                 double *__restrict__ out2)
+                                                 double *__restrict__ out)
 {
   int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.z;
   if (i >= g.nx || j >= g.ny) return;
@@ -1757,23 +1749,17 @@ __global__ __launch_bounds__(256) void k_closure(Geom g, Phys f, int what,
     case 0: out[ip] = vg_sat(pv, f.irg, a, n, f.Sres(ip), f.Ssat(ip)); break;
     case 1: out[ip] = vg_dsat(pv, f.irg, a, n, f.Sres(ip), f.Ssat(ip)); break;
     case 2: out[ip] = vg_kr(pv, f.irg, a, n, f.tb); break;
-    case 3: out[ip] = vg_dkr(pv, f.irg, a, n, f.tb); break;
-    case 4: out[ip] = vg_kr(pv, f.irg, a, n, f.tb) * f.rho; break;
-    default: {
-      double kr = vg_kr(pv, f.irg, a, n, f.tb);
-      out[ip] = kr * f.rho;
-      out2[ip] = vg_dkr(pv, f.irg, a, n, f.tb) * f.rho + kr * 0.0;
-    }
+    default: out[ip] = vg_dkr(pv, f.irg, a, n, f.tb);
   }
 }
 
 static int launch_closure(pfhip_problem *pb, int what, const double *p, double *out,
-                          double *out2, void *stream)
+                          void *stream)
 {
   Geom g = geom_of(pb);
   PROF_BEGIN(PFHIP_PROF_CLOSURE, stream);
   hipLaunchKernelGGL(k_closure, grid3(g), BLOCK3, 0, STREAM(stream), g, phys_of(pb),
-                     what, p, out, out2);
+                     what, p, out);
   PROF_END(PFHIP_PROF_CLOSURE, stream);
   LAUNCHCHK();
   return PFHIP_OK;
@@ -1782,13 +1768,13 @@ static int launch_closure(pfhip_problem *pb, int what, const double *p, double *
 extern "C" int pfhip_saturation(pfhip_problem *pb, const double *p, double *out,
                                 int fcn, void *stream)
 {
-  return launch_closure(pb, fcn == PFHIP_CALCDER ? 1 : 0, p, out, nullptr, stream);
+  return launch_closure(pb, fcn == PFHIP_CALCDER ? 1 : 0, p, out, stream);
 }
 
 extern "C" int pfhip_phase_rel_perm(pfhip_problem *pb, const double *p, double *out,
                                     int fcn, void *stream)
 {
-  return launch_closure(pb, fcn == PFHIP_CALCDER ? 3 : 2, p, out, nullptr, stream);
+  return launch_closure(pb, fcn == PFHIP_CALCDER ? 3 : 2, p, out, stream);
 }
 
 // --------------------------------------------------------------------------
@@ -1963,7 +1949,6 @@ struct ResArgs {
   const double *__restrict__ poro;
   const double *__restrict__ ss;
   const double *__restrict__ src;
-  const double *__restrict__ krho;
   const double *__restrict__ qx;
   const double *__restrict__ qy;
   const double *bcv[6];
@@ -2568,7 +2553,7 @@ static ResArgs res_args(const pfhip_problem *pb, const double *p_old, const doub
   A.p_old = p_old; A.s_old = s_old;
   A.kx = pb->d.kx; A.ky = pb->d.ky; A.kz = pb->d.kz;
   A.poro = pb->d.poro; A.ss = pb->d.ss; A.src = pb->d.src;
-  A.krho = pb->krho; A.qx = pb->q2[0]; A.qy = pb->q2[1];
+  A.qx = pb->q2[0]; A.qy = pb->q2[1];
   for (int f = 0; f < 6; f++) { A.bcv[f] = pb->bcv[f]; A.bct[f] = pb->d.bc[f].type; }
   A.p = nullptr; A.F = nullptr;
   A.pv = nullptr; A.fsub = nullptr; A.pout = nullptr; A.psig = 0.0; A.fsc = 0.0;
@@ -2605,12 +2590,15 @@ extern "C" int pfhip_nl_function_eval(pfhip_problem *pb, const double *p, double
 //   vz[i + nx (j + ny k)]     face k, 0 <= k <= nz
 // Interior faces: the residual's face flux (same operands and order)
 // divided by the face area ffx * z_mult * del_y_slope (= ffx here).
-// One thread per point (i, j, k) of the (nx+1)(ny+1)(nz+1) lattice writes
-// the x, y and z faces on the low side of cell (i, j, k); kr*rho comes from
-// a closure pass into the problem's krho buffer.
-// Algorithmic traffic per cell: p, kr*rho, Kx, Ky, Kz read (40 B) and three
-// velocities written (24 B), plus the closure pass (p, alpha, n read, kr*rho
-// written: 32 B).
+// A cell's thread writes the x, y and z faces on its low side; the domain's
+// own faces come from the shell cells afterwards.  A 64 x 8 tile of columns
+// marches 16 planes: kr*rho of every cell is evaluated once, in place (the
+// tile's west and south neighbours again), the lateral neighbours come from
+// LDS and the lower one from a register.  HBM bounds it: p, alpha, n and K
+// read (32 B isotropic), three velocities written (24 B).  512x512x32: 104 us
+// + 15 us for the domain's faces, 4.5 TB/s (64 x 4 tiles 113 us, 64 x 16
+// 110 us, 32 planes 108 us); a closure pass that stored kr*rho and a pass
+// over the faces took 51 + 139 us.
 // --------------------------------------------------------------------------
 struct VelOut {
   double *__restrict__ vx;
@@ -2618,8 +2606,10 @@ struct VelOut {
   double *__restrict__ vz;
 };
 
-// velocity the BC patch loop of face fc leaves at boundary cell (i, j, k)
-__device__ __forceinline__ double bc_face_velocity(const ResArgs &A, int fc, int i, int j, int k)
+// velocity the BC patch loop of face fc leaves at boundary cell (i, j, k),
+// whose kr*rho is krc (Dirichlet faces)
+__device__ __forceinline__ double bc_face_velocity(const ResArgs &A, int fc, int i, int j, int k,
+                                                   double krc)
 {
   const Geom &g = A.g;
   const double dx = A.dx, dy = A.dy, dz = A.dz, dt = A.dt;
@@ -2631,7 +2621,7 @@ __device__ __forceinline__ double bc_face_velocity(const ResArgs &A, int fc, int
   if (type == PFHIP_BC_FLUX) return value;
   const double pc = A.p[ip];
   if (type == PFHIP_BC_DIR_EQUIL)
-    return dir_u_new(A, fc, ip, value, pc, A.krho[ip], A.kx[ip], A.ky[ip], A.kz[ip]) / h;
+    return dir_u_new(A, fc, ip, value, pc, krc, A.kx[ip], A.ky[ip], A.kz[ip]) / h;
   // OverlandKinematicBC (top face): u_new = h value + q_overlnd / dt
   const double vol = dx * dy * dz;
   const int io = (i + 1) + (j + 1) * g.sy;
@@ -2643,52 +2633,147 @@ __device__ __forceinline__ double bc_face_velocity(const ResArgs &A, int fc, int
   return u_new / h;
 }
 
-__global__ __launch_bounds__(256) void k_face_velocity(ResArgs A, VelOut V)
+#define FVY 8
+#define FVZ 16
+// a / b for a constant b with rb = 1 / b rounded to nearest: the quotient
+// corrected once by its exact remainder, which rounds it as the division does
+// (Markstein, IBM J. Res. Dev. 34 (1990)), in three instructions
+__device__ __forceinline__ double div_const(double a, double b, double rb)
 {
-  const Geom &g = A.g;
-  const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
-  const int k = blockIdx.z;
-  if (i > g.nx || j > g.ny) return;
-  const double *__restrict__ p = A.p;
-  const double *__restrict__ kr = A.krho;
-  const double rho = A.f.rho, grav = A.f.g, mu = A.f.mu;
+  const double q = a * rb;
+  return fma(fma(-b, q, a), rb, q);
+}
+// flux_xy and flux_z over the face area ff: the same operands and order
+__device__ __forceinline__ double vel_xy(double pa, double pb, double ka, double kb, double kra,
+                                         double krb, double ff, double iff, double d, double id,
+                                         double gc, double mu, double imu)
+{
+  const double dd = div_const(pa - pb, d, id);
+  return div_const(div_const(ff * hmean_f(ka, kb) * dd * gc * upw(dd * gc, 0.0, kra, krb), mu,
+                             imu), ff, iff);
+}
+__device__ __forceinline__ double vel_z(double pa, double pb, double ka, double kb, double kra,
+                                        double krb, double ff, double iff, double dz, double idz,
+                                        double hrg, double mu, double imu)
+{
+  const double lc = div_const(pa, dz, idz) - hrg, uc = div_const(pb, dz, idz) + hrg;
+  return div_const(div_const(ff * hmean_f(ka, kb) * (lc - uc) * upw(lc, uc, kra, krb), mu, imu),
+                   ff, iff);
+}
+// a cell's inputs on one plane
+struct VelIn { double p, al, n, kx, ky, kz; };
+
+template <bool ISO>
+__device__ __forceinline__ void load_vel(VelIn &v, const ResArgs &A, int ip)
+{
+  v.p = ldb(A.p, ip); v.al = ldb(A.f.alpha, ip); v.n = ldb(A.f.nvg, ip);
+  v.kz = ldb(A.kz, ip);
+  if constexpr (!ISO) { v.kx = ldb(A.kx, ip); v.ky = ldb(A.ky, ip); }
+  else { v.kx = v.kz; v.ky = v.kz; }
+}
+
+template <bool ISO, bool TAB>
+__global__ __launch_bounds__(64 * FVY) void k_face_velocity(ResArgs A, VelOut V)
+{
+  constexpr int W = 65;                              // the west neighbour, then the tile
+  __shared__ double s_p[2][(FVY + 1) * W], s_kr[2][(FVY + 1) * W], s_k[2][(FVY + 1) * W];
+  __shared__ double s_ky[ISO ? 1 : 2][ISO ? 1 : (FVY + 1) * W];
+  const Geom g = A.g;
+  const Phys &f = A.f;
+  const double rho = f.rho, grav = f.g, mu = f.mu;
   const double dx = A.dx, dy = A.dy, dz = A.dz;
   const double ffx = dy * dz, ffy = dx * dz, ffz = dx * dy;
-  // (i, j, k) may lie one past the last cell in any direction: ip is then
-  // a ghost index, read only by faces that are interior
+  const double iffx = 1.0 / ffx, iffy = 1.0 / ffy, iffz = 1.0 / ffz;
+  const double hrg = 0.5 * rho * grav * 1.0;
+  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
+  int bx, by, bz;
+  tile_of_block(bx, by, bz);
+  const int i = bx * 64 + tx, j = by * FVY + ty;
+  const bool act = i < g.nx && j < g.ny;
+  const int ls = (ty + 1) * W + tx + 1;
+  // loads come from the clamped column
+  const int col = (min(i, g.nx - 1) + 1) + (min(j, g.ny - 1) + 1) * g.sy;
+  // west neighbours (FVY of them), then south ones (64), one per thread
+  int hx = 0, hy = 0;
+  bool halo = false;
+  if (tid < FVY) { hy = tid + 1; halo = bx > 0 && by * FVY + tid < g.ny; }
+  else if (tid < FVY + 64) {
+    hx = tid - FVY + 1;
+    halo = by > 0 && bx * 64 + hx - 1 < g.nx;
+  }
+  const int hcol = halo ? (bx * 64 + hx) + (by * FVY + hy) * g.sy : col;
+  const int hls = hy * W + hx;
+  const int k0 = bz * FVZ, k1 = min(k0 + FVZ, g.nz);
+  double p_m = 0.0, kr_m = 0.0, kz_m = 0.0;
+  if (k0 > 0) {
+    VelIn m;
+    load_vel<ISO>(m, A, col + k0 * g.sz);
+    p_m = m.p;
+    kr_m = vg_kr<TAB>(m.p, f.irg, m.al, m.n, f.tb) * rho;
+    kz_m = m.kz;
+  }
+  VelIn nxt, hn = {};
+  load_vel<ISO>(nxt, A, col + (k0 + 1) * g.sz);
+  if (halo) load_vel<ISO>(hn, A, hcol + (k0 + 1) * g.sz);
+  for (int k = k0; k < k1; k++) {
+    const int q = k & 1;
+    const VelIn c = nxt, h = hn;
+    const int up = (min(k + 1, g.nz - 1) + 1) * g.sz;
+    load_vel<ISO>(nxt, A, col + up);
+    if (halo) load_vel<ISO>(hn, A, hcol + up);
+    const double kr = vg_kr<TAB>(c.p, f.irg, c.al, c.n, f.tb) * rho;
+    s_p[q][ls] = c.p;
+    s_kr[q][ls] = kr;
+    s_k[q][ls] = c.kx;
+    if constexpr (!ISO) s_ky[q][ls] = c.ky;
+    if (halo) {
+      s_p[q][hls] = h.p;
+      s_kr[q][hls] = vg_kr<TAB>(h.p, f.irg, h.al, h.n, f.tb) * rho;
+      s_k[q][hls] = h.kx;
+      if constexpr (!ISO) s_ky[q][hls] = h.ky;
+    }
+    // one barrier a plane: the buffers alternate
+    lds_barrier();
+    if (act) {
+      const double *ky_s = ISO ? s_k[q] : s_ky[ISO ? 0 : q];
+      const long ox = i + (long)(g.nx + 1) * (j + (long)g.ny * k);
+      const long oy = i + (long)g.nx * (j + (long)(g.ny + 1) * k);
+      const long oz = i + (long)g.nx * (j + (long)g.ny * k);
+      const int w = ls - 1, sth = ls - W;
+      if (i > 0)
+        V.vx[ox] = vel_xy(s_p[q][w], c.p, s_k[q][w], c.kx, s_kr[q][w], kr, ffx, iffx, dx, A.idx,
+                          grav, mu, A.imu);
+      if (j > 0)
+        V.vy[oy] = vel_xy(s_p[q][sth], c.p, ky_s[sth], c.ky, s_kr[q][sth], kr, ffy, iffy, dy,
+                          A.idy, grav, mu, A.imu);
+      if (k > 0)
+        V.vz[oz] = vel_z(p_m, c.p, kz_m, c.kz, kr_m, kr, ffz, iffz, dz, A.idz, hrg, mu, A.imu);
+    }
+    p_m = c.p; kr_m = kr; kz_m = c.kz;
+  }
+}
+
+// the domain's faces, from the shell cells (inside the tiled kernel their
+// code cost it scalar-register spills in every plane)
+__global__ __launch_bounds__(256) void k_face_velocity_bc(ResArgs A, VelOut V, long nshell)
+{
+  const Geom &g = A.g;
+  const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  int i, j, k;
+  if (c >= nshell || !shell_cell(g, c, i, j, k)) return;
   const int ip = (i + 1) + (j + 1) * g.sy + (k + 1) * g.sz;
-  if (j < g.ny && k < g.nz) {
-    double v;
-    if (i == 0) v = bc_face_velocity(A, 0, 0, j, k);
-    else if (i == g.nx) v = bc_face_velocity(A, 1, g.nx - 1, j, k);
-    else {
-      const int a = ip - 1;
-      v = flux_xy(p[a], p[ip], A.kx[a], A.kx[ip], kr[a], kr[ip], ffx, dx, grav, mu) /
-          (ffx * 1.0 * 1.0);
-    }
-    V.vx[i + (long)(g.nx + 1) * (j + (long)g.ny * k)] = v;
-  }
-  if (i < g.nx && k < g.nz) {
-    double v;
-    if (j == 0) v = bc_face_velocity(A, 2, i, 0, k);
-    else if (j == g.ny) v = bc_face_velocity(A, 3, i, g.ny - 1, k);
-    else {
-      const int a = ip - g.sy;
-      v = flux_xy(p[a], p[ip], A.ky[a], A.ky[ip], kr[a], kr[ip], ffy, dy, grav, mu) /
-          (ffy * 1.0 * 1.0);
-    }
-    V.vy[i + (long)g.nx * (j + (long)(g.ny + 1) * k)] = v;
-  }
-  if (i < g.nx && j < g.ny) {
-    double v;
-    if (k == 0) v = bc_face_velocity(A, 4, i, j, 0);
-    else if (k == g.nz) v = bc_face_velocity(A, 5, i, j, g.nz - 1);
-    else {
-      const int a = ip - g.sz;
-      v = flux_z(p[a], p[ip], A.kz[a], A.kz[ip], kr[a], kr[ip], ffz, dz, rho, grav, mu) /
-          (ffz * 1.0 * 1.0);
-    }
-    V.vz[i + (long)g.nx * (j + (long)g.ny * k)] = v;
+  const double krc = vg_kr(A.p[ip], A.f.irg, A.f.alpha[ip], A.f.nvg[ip], A.f.tb) * A.f.rho;
+#pragma unroll 1
+  for (int fc = 0; fc < 6; fc++) {
+    const bool on = (fc == 0 && i == 0) || (fc == 1 && i == g.nx - 1) ||
+                    (fc == 2 && j == 0) || (fc == 3 && j == g.ny - 1) ||
+                    (fc == 4 && k == 0) || (fc == 5 && k == g.nz - 1);
+    if (!on) continue;
+    const int hi = fc & 1;
+    const double v = bc_face_velocity(A, fc, i, j, k, krc);
+    if (fc < 2) V.vx[i + hi + (long)(g.nx + 1) * (j + (long)g.ny * k)] = v;
+    else if (fc < 4) V.vy[i + (long)g.nx * (j + hi + (long)(g.ny + 1) * k)] = v;
+    else V.vz[i + (long)g.nx * (j + (long)g.ny * (k + hi))] = v;
   }
 }
 
@@ -2710,14 +2795,19 @@ extern "C" int pfhip_face_velocity(pfhip_problem *pb, const double *p, const dou
                        pb->q2[1]);
     LAUNCHCHK();
   }
-  int rc = launch_closure(pb, 4, p, pb->krho, nullptr, stream);
-  if (rc) return rc;
   ResArgs A = res_args(pb, p_old, nullptr, dt);
   A.p = p;
   VelOut V;
   V.vx = vx; V.vy = vy; V.vz = vz;
-  dim3 grid((g.nx + 1 + 63) / 64, (g.ny + 1 + 3) / 4, g.nz + 1);
-  hipLaunchKernelGGL(k_face_velocity, grid, dim3(64, 4, 1), 0, st, A, V);
+  const dim3 grid((g.nx + 63) / 64, (g.ny + FVY - 1) / FVY, (g.nz + FVZ - 1) / FVZ);
+  const dim3 block(64, FVY, 1);
+  const bool iso = A.kx == A.ky && A.kx == A.kz;
+  if (A.f.tb.t) hipLaunchKernelGGL((k_face_velocity<false, true>), grid, block, 0, st, A, V);
+  else if (iso) hipLaunchKernelGGL((k_face_velocity<true, false>), grid, block, 0, st, A, V);
+  else hipLaunchKernelGGL((k_face_velocity<false, false>), grid, block, 0, st, A, V);
+  const long ns = shell_count(g);
+  hipLaunchKernelGGL(k_face_velocity_bc, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, st, A,
+                     V, ns);
   LAUNCHCHK();
   return PFHIP_OK;
 }
@@ -2738,43 +2828,50 @@ extern "C" int pfhip_face_velocity(pfhip_problem *pb, const double *p, const dou
 //   dM_sub + dM_surf = [0] + [1] - [2] + [3]
 // with dM_sub the change of ParFlow's own stored mass (the residual's
 // accumulation terms) and dM_surf that of the surface storage
-// dx dy max(p_top, 0).  Row-owning blocks and a fixed-order final pass.
+// dx dy max(p_top, 0).  The faces belong to the shell cells, so only those
+// are visited (kr*rho of the Dirichlet ones evaluated in place), and all
+// cells only for a source field; fixed mapping, fixed-order final pass.
 // --------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_wb_terms(ResArgs A, int overland,
+__global__ __launch_bounds__(256) void k_wb_terms(ResArgs A, int overland, long nshell,
                                                   double *__restrict__ partial, int nb)
 {
   const Geom &g = A.g;
   const double dx = A.dx, dy = A.dy, dz = A.dz, dt = A.dt;
   const double vol_time = dx * dy * dz * dt;
   double bin = 0.0, rain = 0.0, run = 0.0, src = 0.0;
-  const int rows = g.ny * g.nz;
-  for (int r = blockIdx.x; r < rows; r += gridDim.x) {
-    const int j = r % g.ny, k = r / g.ny;
-    const int base = 1 + (j + 1) * g.sy + (k + 1) * g.sz;
-    for (int i = threadIdx.x; i < g.nx; i += blockDim.x) {
-      const int ip = base + i;
-      if (A.src) src += A.src[ip] * vol_time;
-      const bool bnd = (i == 0) | (i == g.nx - 1) | (j == 0) | (j == g.ny - 1) | (k == 0) |
-                       (k == g.nz - 1);
-      if (!bnd) continue;
-      for (int fc = 0; fc < 6; fc++) {
-        const bool on = (fc == 0 && i == 0) || (fc == 1 && i == g.nx - 1) ||
-                        (fc == 2 && j == 0) || (fc == 3 && j == g.ny - 1) ||
-                        (fc == 4 && k == 0) || (fc == 5 && k == g.nz - 1);
-        if (!on) continue;
-        const double dir = (fc & 1) ? 1.0 : -1.0;
-        const double h = (fc < 2) ? dy * dz : (fc < 4) ? dx * dz : dx * dy;
-        if (fc == 5 && overland) {
-          const int fi = i + j * g.nx;
-          rain += -dt * (h * A.bcv[5][fi]);
-          const int io = (i + 1) + (j + 1) * g.sy;
-          if (i == g.nx - 1) run += dt * dy * A.qx[io];
-          if (i == 0) run -= dt * dy * A.qx[io - 1];
-          if (j == g.ny - 1) run += dt * dx * A.qy[io];
-          if (j == 0) run -= dt * dx * A.qy[io - g.sy];
-        } else {
-          bin += -dt * dir * h * bc_face_velocity(A, fc, i, j, k);
+  if (A.src) {
+    const int rows = g.ny * g.nz;
+    for (int r = blockIdx.x; r < rows; r += gridDim.x) {
+      const int base = 1 + (r % g.ny + 1) * g.sy + (r / g.ny + 1) * g.sz;
+      for (int i = threadIdx.x; i < g.nx; i += blockDim.x) src += A.src[base + i] * vol_time;
+    }
+  }
+  const long step = (long)gridDim.x * blockDim.x;
+  for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < nshell; c += step) {
+    int i, j, k;
+    if (!shell_cell(g, c, i, j, k)) break;
+    for (int fc = 0; fc < 6; fc++) {
+      const bool on = (fc == 0 && i == 0) || (fc == 1 && i == g.nx - 1) ||
+                      (fc == 2 && j == 0) || (fc == 3 && j == g.ny - 1) ||
+                      (fc == 4 && k == 0) || (fc == 5 && k == g.nz - 1);
+      if (!on) continue;
+      const double dir = (fc & 1) ? 1.0 : -1.0;
+      const double h = (fc < 2) ? dy * dz : (fc < 4) ? dx * dz : dx * dy;
+      if (fc == 5 && overland) {
+        const int fi = i + j * g.nx;
+        rain += -dt * (h * A.bcv[5][fi]);
+        const int io = (i + 1) + (j + 1) * g.sy;
+        if (i == g.nx - 1) run += dt * dy * A.qx[io];
+        if (i == 0) run -= dt * dy * A.qx[io - 1];
+        if (j == g.ny - 1) run += dt * dx * A.qy[io];
+        if (j == 0) run -= dt * dx * A.qy[io - g.sy];
+      } else {
+        double krc = 0.0;
+        if (A.bct[fc] == PFHIP_BC_DIR_EQUIL) {
+          const int ip = (i + 1) + (j + 1) * g.sy + (k + 1) * g.sz;
+          krc = vg_kr(A.p[ip], A.f.irg, A.f.alpha[ip], A.f.nvg[ip], A.f.tb) * A.f.rho;
         }
+        bin += -dt * dir * h * bc_face_velocity(A, fc, i, j, k, krc);
       }
     }
   }
@@ -2809,15 +2906,15 @@ extern "C" int pfhip_water_balance_fluxes(pfhip_problem *pb, const double *p,
                        pb->q2[1]);
     LAUNCHCHK();
   }
-  int rc = launch_closure(pb, 4, p, pb->krho, nullptr, stream);
-  if (rc) return rc;
   ResArgs A = res_args(pb, p_old, nullptr, dt);
   A.p = p;
-  int nb = red_blocks(g);
-  hipLaunchKernelGGL(k_wb_terms, dim3(nb), dim3(256), 0, st, A, pb->overland ? 1 : 0,
+  const long ns = shell_count(g);
+  const long want = (ns + 255) / 256;
+  const int nb = pb->d.src || want > red_blocks(g) ? red_blocks(g) : (int)want;
+  hipLaunchKernelGGL(k_wb_terms, dim3(nb), dim3(256), 0, st, A, pb->overland ? 1 : 0, ns,
                      pb->red_partial, nb);
   LAUNCHCHK();
-  rc = red_fetch(pb, nb, PFHIP_WB_TERMS, 0, 0, PFHIP_WB_TERMS, stream);
+  const int rc = red_fetch(pb, nb, PFHIP_WB_TERMS, 0, 0, PFHIP_WB_TERMS, stream);
   if (rc) return rc;
   for (int q = 0; q < PFHIP_WB_TERMS; q++) out[q] = pb->h_red[q];
   return PFHIP_OK;
@@ -3100,8 +3197,6 @@ struct JacArgs {
   const double *__restrict__ kz;
   const double *__restrict__ poro;
   const double *__restrict__ ss;
-  const double *__restrict__ krho;
-  const double *__restrict__ dkrho;
   const double *__restrict__ ke;
   const double *__restrict__ kw;
   const double *__restrict__ kn;
@@ -3551,7 +3646,6 @@ int pfhip_jacobian_into(pfhip_problem *pb, const double *p, double dt, int symm,
   A.p = p;
   A.kx = pb->d.kx; A.ky = pb->d.ky; A.kz = pb->d.kz;
   A.poro = pb->d.poro; A.ss = pb->d.ss;
-  A.krho = nullptr; A.dkrho = nullptr;
   A.ke = pb->q2[0]; A.kw = pb->q2[1]; A.kn = pb->q2[2]; A.ks = pb->q2[3];
   for (int f = 0; f < 6; f++) { A.bcv[f] = pb->bcv[f]; A.bct[f] = pb->d.bc[f].type; }
   A.symm = symm;
@@ -4157,7 +4251,6 @@ extern "C" int pfhip_ens_exec_jacobian(pfhip_ens_req *const *rq, int n, pfhip_en
     A.p = q->x;
     A.kx = pb->d.kx; A.ky = pb->d.ky; A.kz = pb->d.kz;
     A.poro = pb->d.poro; A.ss = pb->d.ss;
-    A.krho = nullptr; A.dkrho = nullptr;
     A.ke = A.kw = A.kn = A.ks = nullptr;
     for (int f = 0; f < 6; f++) { A.bcv[f] = pb->bcv[f]; A.bct[f] = pb->d.bc[f].type; }
     A.symm = 1;

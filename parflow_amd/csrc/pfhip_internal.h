@@ -20,7 +20,6 @@ struct pfhip_problem {
   int overland;               /* top face is OverlandKinematic            */
   double *bcv[6];             /* device per-face BC values                */
   double *h_bcv[6];           /* pinned host staging                      */
-  double *krho, *dkrho;       /* device scratch, ghosted                  */
   double *q2[4];              /* device surface scratch                   */
   double *red_partial;        /* reduction partials (RED_MAX_BLOCKS*8)    */
   double *red_dev;            /* device result slots (PFHIP_RED_SLOTS)    */

@@ -50,3 +50,47 @@ def test_reduction_results_reach_the_host(gpu, shape):
                                                      C.byref(b), None), "dot_scsteplength")
             assert abs(a.value - np.sum(Y * Y)) <= 1e-13 * np.sum(Y * Y)
             assert abs(b.value - np.max(np.abs(Y) / (1 + np.abs(X)))) <= 1e-15 * b.value
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (64, 8, 16), (65, 9, 17), (130, 3, 33)])
+@pytest.mark.parametrize("overland,dirs", [(False, True), (True, False)])
+def test_face_velocity_tiles(gpu, shape, overland, dirs):
+    """Face velocities over grids that fill, exceed and fall short of the
+    kernel's 64 x 8 x 16 tiles, against the oracle."""
+    api = _api()
+    prob = cases.hetero(*shape, seed=4, overland=overland, dir_sides=dirs)
+    gp, op = api.GPUProblem(prob), O.OracleProblem(prob)
+    p, p_old = cases.random_pressure(prob, seed=5), cases.random_pressure(prob, seed=6)
+    t = 0.1
+    got = gp.face_velocity(p, p_old, 0.1, t)
+    want = O.face_velocity(op, p, p_old, 0.1, t)
+    scale = max(np.max(np.abs(b)) for b in want)
+    for a, b in zip(got, want):
+        assert np.max(np.abs(a - b)) <= 1e-12 * scale
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 2, 2), (70, 9, 5)])
+@pytest.mark.parametrize("with_src", [False, True])
+def test_water_balance_fluxes_shell(gpu, shape, with_src):
+    """The step's volumes from the shell cells alone (and all cells of a
+    source field), against the face velocities summed over the domain."""
+    api = _api()
+    prob = cases.hetero(*shape, seed=8, dir_sides=True)
+    src = cases.hetero_src(prob, 9) if with_src else None
+    gp = api.GPUProblem(prob, src=src)
+    p = cases.random_pressure(prob, seed=10)
+    dt, t = 0.1, 0.1
+    f = gp.water_balance_fluxes(p, p, dt, t)
+    vx, vy, vz = O.face_velocity(O.OracleProblem(prob), p, p, dt, t)
+    ax, ay, az = prob.dy * prob.dz, prob.dx * prob.dz, prob.dx * prob.dy
+    terms = [ax * vx[:, :, 0], -ax * vx[:, :, -1], ay * vy[:, 0], -ay * vy[:, -1],
+             az * vz[0], -az * vz[-1]]
+    want = dt * sum(float(np.sum(a)) for a in terms)
+    scale = dt * sum(float(np.sum(np.abs(a))) for a in terms)
+    assert abs(f[0] - want) <= 1e-12 * scale
+    vol = prob.dx * prob.dy * prob.dz * dt
+    if with_src:
+        want = vol * float(np.sum(prob.interior(src)))
+        assert abs(f[3] - want) <= 1e-12 * vol * float(np.sum(np.abs(src)))
+    else:
+        assert f[3] == 0.0
