@@ -2157,7 +2157,7 @@ __device__ __forceinline__ double flux_z_i(double pa, double pb, double ka, doub
 }
 
 // Software-pipelined fused residual.  A TX x TY block owns a tile of
-// columns and marches up a z-chunk of ZC planes; each cell computes its
+// columns and marches up a z-chunk of zc planes; each cell computes its
 // closures one plane ahead and the fluxes through its own x+, y+, z+ faces
 // once (the tile's west/south edge halo is recomputed); every global load of plane k+1
 // (k+2 for the closure inputs) is issued at the top of plane k from a
@@ -2243,8 +2243,8 @@ __device__ __forceinline__ void load_hal(HalIn &h, const ResArgs &A, int hip, do
   h.p = p_at<MODE>(A, hip, psig); h.al = ldb(A.f.alpha, hip); h.n = ldb(A.f.nvg, hip);
 }
 
-template <int TX, int TY, int ZC, bool PCS, int MODE, bool ISO, bool TAB>
-__global__ __launch_bounds__(TX * TY) void k_residual_pf(ResArgs A)
+template <int TX, int TY, bool PCS, int MODE, bool ISO, bool TAB>
+__global__ __launch_bounds__(TX * TY) void k_residual_pf(ResArgs A, int zc)
 {
   constexpr int HALO = 2 * TX + 2 * TY;
   constexpr int W2 = TX + 2;
@@ -2292,8 +2292,8 @@ __global__ __launch_bounds__(TX * TY) void k_residual_pf(ResArgs A)
   const bool hw0 = tid < HALO && hx == 0, hs0 = tid < HALO && hy == 0;
   const double *__restrict__ Kh = ISO ? A.kz : hsouth ? A.ky : A.kx;
   const int hoff = hsouth ? sy : 1;
-  const int k0 = bz * ZC;
-  const int k1 = min(k0 + ZC, nz);
+  const int k0 = bz * zc;
+  const int k1 = min(k0 + zc, nz);
   auto plane = [&](int q) { return (min(q, nz - 1) + 1) * sz; };
 
   double p_m = 0, kr_m = 0, kz_m = 0;
@@ -2495,19 +2495,38 @@ __global__ __launch_bounds__(256) void k_residual_bc(ResArgs A, long nshell)
   }
 }
 
-// launch geometry of the tiled residual (launch_residual's 64 x 8 x 16
-// tiles) and of the boundary-shell kernel
+// launch geometry of the tiled residual and Jacobian (64 x 8 columns,
+// res_zc planes) and of the boundary-shell kernel
+//
+// A tile marches its planes one after another, so on a small grid the time is
+// that march's and not the chip's.  16 planes where that makes the 512 tiles
+// that are resident at once (256 CUs, two tiles each); fewer, down to 2, until
+// there are as many (a chunk evaluates one plane of closures twice).  F and
+// the symmetric Jacobian with 16 planes and with the rule's: 32^3 45 and
+// 51 us -> 15 and 15 (2 planes), 131x97x25 42 and 48 -> 21 and 22 (2),
+// 256x256x16 43 and 46 -> 27 and 28 (4).  A bound of 256 tiles takes 30 and
+// 32 us on 256x256x16; one of 1024 costs 256x256x64 2 to 5 %.
+#define RES_FILL 512
+static int res_zc(const Geom &g)
+{
+  const long cols = (long)((g.nx + 63) / 64) * ((g.ny + 7) / 8);
+  int zc = 16;
+  while (zc > 2 && cols * ((g.nz + zc - 1) / zc) < RES_FILL) zc /= 2;
+  return zc;
+}
 static long res_tiles(const Geom &g)
 {
-  return (long)((g.nx + 63) / 64) * ((g.ny + 7) / 8) * ((g.nz + 15) / 16);
+  const int zc = res_zc(g);
+  return (long)((g.nx + 63) / 64) * ((g.ny + 7) / 8) * ((g.nz + zc - 1) / zc);
 }
 static long res_bc_blocks(const Geom &g) { return (shell_count(g) + 255) / 256; }
 
-template <int TX, int TY, int ZC, int MODE>
+template <int TX, int TY, int MODE>
 static void launch_pf(const ResArgs &A, hipStream_t st)
 {
   const Geom &g = A.g;
-  dim3 grid((g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, (g.nz + ZC - 1) / ZC);
+  const int zc = res_zc(g);
+  dim3 grid((g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, (g.nz + zc - 1) / zc);
   dim3 block(TX, TY, 1);
   const int pid = (MODE == 1) ? PFHIP_PROF_RESIDUAL_JV
                   : (MODE == 2) ? PFHIP_PROF_RESIDUAL_STEP : PFHIP_PROF_RESIDUAL;
@@ -2516,15 +2535,15 @@ static void launch_pf(const ResArgs &A, hipStream_t st)
   if (A.f.tb.t) {
     // kr from a lookup table: the general (anisotropic) form
     if (A.f.sres || A.f.ssat)
-      hipLaunchKernelGGL((k_residual_pf<TX, TY, ZC, true, MODE, false, true>), grid, block, 0, st, A);
+      hipLaunchKernelGGL((k_residual_pf<TX, TY, true, MODE, false, true>), grid, block, 0, st, A, zc);
     else
-      hipLaunchKernelGGL((k_residual_pf<TX, TY, ZC, false, MODE, false, true>), grid, block, 0, st, A);
+      hipLaunchKernelGGL((k_residual_pf<TX, TY, false, MODE, false, true>), grid, block, 0, st, A, zc);
   } else if (A.f.sres || A.f.ssat) {
-    if (iso) hipLaunchKernelGGL((k_residual_pf<TX, TY, ZC, true, MODE, true, false>), grid, block, 0, st, A);
-    else hipLaunchKernelGGL((k_residual_pf<TX, TY, ZC, true, MODE, false, false>), grid, block, 0, st, A);
+    if (iso) hipLaunchKernelGGL((k_residual_pf<TX, TY, true, MODE, true, false>), grid, block, 0, st, A, zc);
+    else hipLaunchKernelGGL((k_residual_pf<TX, TY, true, MODE, false, false>), grid, block, 0, st, A, zc);
   } else {
-    if (iso) hipLaunchKernelGGL((k_residual_pf<TX, TY, ZC, false, MODE, true, false>), grid, block, 0, st, A);
-    else hipLaunchKernelGGL((k_residual_pf<TX, TY, ZC, false, MODE, false, false>), grid, block, 0, st, A);
+    if (iso) hipLaunchKernelGGL((k_residual_pf<TX, TY, false, MODE, true, false>), grid, block, 0, st, A, zc);
+    else hipLaunchKernelGGL((k_residual_pf<TX, TY, false, MODE, false, false>), grid, block, 0, st, A, zc);
   }
   PROF_END(pid, st);
   long ns = shell_count(g);
@@ -2535,9 +2554,9 @@ static void launch_pf(const ResArgs &A, hipStream_t st)
 static void launch_residual(const ResArgs &A, hipStream_t st)
 {
   const int mode = (A.pv == nullptr) ? 0 : (A.fsub != nullptr) ? 1 : 2;
-  if (mode == 1) launch_pf<64, 8, 16, 1>(A, st);
-  else if (mode == 2) launch_pf<64, 8, 16, 2>(A, st);
-  else launch_pf<64, 8, 16, 0>(A, st);
+  if (mode == 1) launch_pf<64, 8, 1>(A, st);
+  else if (mode == 2) launch_pf<64, 8, 2>(A, st);
+  else launch_pf<64, 8, 0>(A, st);
 }
 
 // the problem-fixed part of the residual arguments; the caller sets the
@@ -3303,11 +3322,11 @@ __device__ __forceinline__ void jface_z(double pa, double pb, double ka, double 
   T2 = zc * (diff * upw(lc, uc, 0.0, dkb)) + sym_u;
 }
 
-template <int TX, int TY, int ZC, bool PCS, bool SYMM, typename OT, bool TAB>
+template <int TX, int TY, bool PCS, bool SYMM, typename OT, bool TAB>
 // four waves per SIMD: the register budget of 128 VGPRs (without the hint
 // the compiler took 131 and three waves; 401 -> 328 us on 16.8M cells)
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(4)))
-void k_jacobian_pf(JacPFArgs P, JOut<OT> J)
+void k_jacobian_pf(JacPFArgs P, JOut<OT> J, int zc)
 {
   constexpr int HALO = 2 * TX + 2 * TY;
   constexpr int W2 = TX + 2;
@@ -3354,8 +3373,8 @@ void k_jacobian_pf(JacPFArgs P, JOut<OT> J)
   const bool hsouth = hact && hy == 0;
   const double *__restrict__ Kh = hsouth ? A.ky : A.kx;
   const int hoff = hsouth ? sy : 1;
-  const int k0 = bz * ZC;
-  const int k1 = min(k0 + ZC, nz);
+  const int k0 = bz * zc;
+  const int k1 = min(k0 + zc, nz);
   auto plane = [&](int q) { return (min(q, nz - 1) + 1) * sz; };
 
   double p_c = 0, S_c = 0, dS_c = 0, kr_c = 0, dk_c = 0, kz_c = 0;
@@ -3608,17 +3627,18 @@ template <bool SYMM, typename OT>
 static void launch_jacobian_pf(const JacPFArgs &P, const JOut<OT> &J, hipStream_t st)
 {
   const Geom &g = P.a.g;
-  constexpr int TX = 64, TY = 8, ZC = 16;
-  dim3 grid((g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, (g.nz + ZC - 1) / ZC);
+  constexpr int TX = 64, TY = 8;
+  const int zc = res_zc(g);
+  dim3 grid((g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, (g.nz + zc - 1) / zc);
   dim3 block(TX, TY, 1);
   PROF_BEGIN(PFHIP_PROF_JACOBIAN, st);
   const bool tab = P.a.f.tb.t != nullptr;
   if (P.a.f.sres || P.a.f.ssat) {
-    if (tab) hipLaunchKernelGGL((k_jacobian_pf<TX, TY, ZC, true, SYMM, OT, true>), grid, block, 0, st, P, J);
-    else hipLaunchKernelGGL((k_jacobian_pf<TX, TY, ZC, true, SYMM, OT, false>), grid, block, 0, st, P, J);
+    if (tab) hipLaunchKernelGGL((k_jacobian_pf<TX, TY, true, SYMM, OT, true>), grid, block, 0, st, P, J, zc);
+    else hipLaunchKernelGGL((k_jacobian_pf<TX, TY, true, SYMM, OT, false>), grid, block, 0, st, P, J, zc);
   } else {
-    if (tab) hipLaunchKernelGGL((k_jacobian_pf<TX, TY, ZC, false, SYMM, OT, true>), grid, block, 0, st, P, J);
-    else hipLaunchKernelGGL((k_jacobian_pf<TX, TY, ZC, false, SYMM, OT, false>), grid, block, 0, st, P, J);
+    if (tab) hipLaunchKernelGGL((k_jacobian_pf<TX, TY, false, SYMM, OT, true>), grid, block, 0, st, P, J, zc);
+    else hipLaunchKernelGGL((k_jacobian_pf<TX, TY, false, SYMM, OT, false>), grid, block, 0, st, P, J, zc);
   }
   PROF_END(PFHIP_PROF_JACOBIAN, st);
   long ns = shell_count(g);

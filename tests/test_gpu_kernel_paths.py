@@ -94,3 +94,24 @@ def test_water_balance_fluxes_shell(gpu, shape, with_src):
         assert abs(f[3] - want) <= 1e-12 * vol * float(np.sum(np.abs(src)))
     else:
         assert f[3] == 0.0
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (64, 8, 2), (65, 9, 3), (200, 130, 9), (513, 130, 35)])
+def test_residual_and_jacobian_plane_chunks(gpu, shape):
+    """F and both Jacobians where the tiles march 2, 4 and 8 planes and the
+    last chunk is cut short, against the oracle."""
+    api = _api()
+    prob = cases.hetero(*shape, seed=11, dir_sides=True)
+    gp, op = api.GPUProblem(prob), O.OracleProblem(prob)
+    p, p_old = cases.random_pressure(prob, seed=12), cases.random_pressure(prob, seed=13)
+    s_old = O.saturation(op, p_old, 0)
+    I = prob.interior
+    a = I(gp.nl_function_eval(p, p_old, s_old, 0.1, 0.1))
+    b = I(O.nl_function_eval(op, p, p_old, s_old, 0.1, 0.1))
+    assert np.max(np.abs(a - b)) <= 1e-12 * np.max(np.abs(b))
+    for symm in (0, 1):
+        A = gp.richards_jacobian_eval(p, 0.1, 0.1, symm)
+        B = O.jacobian_eval(op, p, 0.1, 0.1, symm)
+        scale = np.max(np.abs(I(B[0])))
+        for q in ((0, 2, 4, 6) if symm else range(7)):
+            assert np.max(np.abs(I(A[q]) - I(B[q]))) <= 1e-11 * scale, (symm, q)
