@@ -1524,98 +1524,366 @@ __global__ __launch_bounds__(CWG) void k_coarse_vcycle(const LevelDev<T> *__rest
 }
 
 // The same bottom with every level's arrays in LDS (symmetric storage).
-// Each level is copied into a compact, ghost-free block of LDS (C, E, N,
-// U, x, b, t, p1, p2 of its points); its LDS level record carries compact
-// strides and array pointers shifted so that LIDX addresses the compact
-// block.  Every per-point function reads a neighbour or a lower coupling
-// only when that neighbour exists, so no ghost entry is ever touched.  The
-// phases then wait on LDS instead of L2, and the sweeps, residuals and
-// transfers are the global kernel's (the same functions, in the same
-// order).  b of the top level is copied in, x of the top level out; the
-// coarser levels' x, b, t are produced inside.
+// Each level is copied into a compact, ghost-free block of LDS (C, E, N, U,
+// x, b, t, p1, p2 of its points).  b of the top level is copied in, x of the
+// top level out; the coarser levels' x, b, t are produced inside.  The sweeps,
+// residuals and transfers are the global kernel's, point by point in the same
+// order.
+//
+// A dozen levels with ten phases each make this a chain of short phases, so
+// the work between two barriers is what counts:
+//   * a thread owns the pair of x-neighbours (2m, 2m+1) of a row, one red and
+//     one black point; their rows, b and the places of the neighbours' x stay
+//     in registers through a visit of the level, and a half-sweep reads six
+//     values of x (the index divisions are per visit, by multiplication);
+//   * the level's sizes come in scalar registers, and every access is an LDS
+//     instruction at an offset from the block's base (pointers kept in a
+//     level record made them flat accesses);
+//   * levels of at most 64 pairs run in the first wavefront alone, without
+//     workgroup barriers;
+//   * the copy-in issues the loads of all levels together.
+// The last 12 levels of 512x512x64 in FP32, 2 + 2 sweeps: 124 -> 55 us; the
+// last 11 of 32^3 in FP64, 1 + 1 sweeps: 67 -> 39 us (was one point per thread
+// with the level records and their pointers in LDS).
 #define LDS_ALIGN 16
-__host__ __device__ static inline long lds_level_table_bytes(int nl, long rec)
+
+// what the LDS bottom reads of a level: host-built, uniform, so it arrives in
+// scalar registers
+template <typename T> struct BLevel {
+  int n[3], dir;
+  int s1, s2;                 // compact strides
+  int gs1, gs2;               // ghosted strides
+  unsigned cum;               // points of the finer levels
+  int np, ncol, npair;        // points, pairs of a row, pairs
+  unsigned mcol, mrow;        // ceil(2^32 / ncol), ceil(2^32 / n[1]); 0 for 1
+  const T *g[6], *gb;         // C, E, N, U, p1, p2 and b in global memory
+};
+enum { BQ_C = 0, BQ_E = 1, BQ_N = 2, BQ_U = 3, BQ_P1 = 4, BQ_P2 = 5, BQ_X = 6, BQ_B = 7, BQ_T = 8 };
+
+// q / d and its remainder by the level's multiplier (exact: q d < 2^32)
+__device__ __forceinline__ int b_div(int q, int d, unsigned m, int &rem)
 {
-  return ((nl * rec) + LDS_ALIGN - 1) & ~(long)(LDS_ALIGN - 1);
+  const int r = m ? (int)__umulhi((unsigned)q, m) : q;
+  rem = q - r * d;
+  return r;
+}
+
+// a point of the visited level: its index there (-1: none), its row and where
+// its neighbours' x are in the pool (the zero word where there is none, with
+// a zero coupling)
+template <typename T> struct BPoint {
+  int ip;
+  T c, b, aw, ae, as, an, al, au;
+  int xw, xe, xs, xn, xl, xu;
+};
+template <typename T> struct BPair { BPoint<T> p[2]; };   // [1] red, [0] black
+
+template <typename T>
+__device__ __forceinline__ void b_point(BPoint<T> &P, const T *pool, const BLevel<T> &L, int off,
+                                        int i, int j, int k)
+{
+  const bool in = i < L.n[0];
+  const int ip = (in ? i : 0) + j * L.s1 + k * L.s2, np = L.np;
+  const bool hw = in && i > 0, he = i + 1 < L.n[0], hs = j > 0, hn = j + 1 < L.n[1];
+  const bool hl = k > 0, hu = k + 1 < L.n[2];
+  // offsets from the pool's start, whose first word is zero; the loads are
+  // unconditional (behind a branch each would wait alone)
+  const int c = off + ip, x = off + BQ_X * np + ip;
+  P.ip = in ? ip : -1;
+  P.c = pool[c + BQ_C * np];
+  P.b = pool[c + BQ_B * np];
+  P.aw = pool[hw ? c + BQ_E * np - 1 : 0];
+  P.ae = pool[he ? c + BQ_E * np : 0];
+  P.as = pool[hs ? c + BQ_N * np - L.s1 : 0];
+  P.an = pool[hn ? c + BQ_N * np : 0];
+  P.al = pool[hl ? c + BQ_U * np - L.s2 : 0];
+  P.au = pool[hu ? c + BQ_U * np : 0];
+  P.xw = hw ? x - 1 : 0; P.xe = he ? x + 1 : 0;
+  P.xs = hs ? x - L.s1 : 0; P.xn = hn ? x + L.s1 : 0;
+  P.xl = hl ? x - L.s2 : 0; P.xu = hu ? x + L.s2 : 0;
+}
+
+// pair q of a level: the red point ((i + j + k) odd) and the black one
+template <typename T>
+__device__ __forceinline__ void b_pair(BPair<T> &P, const T *pool, const BLevel<T> &L, int off,
+                                       int m, int j, int k)
+{
+  const int odd = (j + k) & 1;
+  b_point(P.p[1], pool, L, off, 2 * m + (odd ^ 1), j, k);
+  b_point(P.p[0], pool, L, off, 2 * m + odd, j, k);
+}
+
+// gs_update of a visited point; an absent neighbour's product is 0 times 0,
+// and the products are rounded one by one as gs_update's selects leave them
+template <typename T>
+__device__ __forceinline__ void b_half(const BPoint<T> &P, T *pool, T *X, int init)
+{
+#pragma clang fp contract(off)
+  T v;
+  if (init) {
+    v = gs_div(P.b, P.c);
+  } else {
+    const T w = P.aw * pool[P.xw], e = P.ae * pool[P.xe];
+    const T so = P.as * pool[P.xs], no = P.an * pool[P.xn];
+    const T lo = P.al * pool[P.xl], up = P.au * pool[P.xu];
+    const T sum = w + e + so + no + lo + up;
+    v = gs_div(P.b - sum, P.c);
+  }
+  if (P.ip >= 0) X[P.ip] = v;
+}
+
+__device__ __forceinline__ float b_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double b_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// resid_point's b - A x of a visited point into R
+template <typename T>
+__device__ __forceinline__ void b_resid(const BPoint<T> &P, const T *pool, const T *X, T *R)
+{
+  T v = P.c * X[max(P.ip, 0)];
+  v = b_fma(P.aw, pool[P.xw], v);
+  v = b_fma(P.ae, pool[P.xe], v);
+  v = b_fma(P.as, pool[P.xs], v);
+  v = b_fma(P.an, pool[P.xn], v);
+  v = b_fma(P.al, pool[P.xl], v);
+  v = b_fma(P.au, pool[P.xu], v);
+  if (P.ip >= 0) R[P.ip] = P.b - v;
+}
+
+// between two phases: the workgroup, or the one wavefront that runs a small
+// level (its LDS operations complete in order)
+template <bool WAVE> __device__ __forceinline__ void b_sync()
+{
+  if (WAVE) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    lds_barrier();
+  }
+}
+
+// RedBlackGSPoint's call sequence (rbgs_block) on a visited level
+template <typename T, bool WAVE>
+__device__ __forceinline__ void b_sweeps(T *pool, const BLevel<T> &L, int off, const BPair<T> &P,
+                                         int zero, int max_iter, int symmetric)
+{
+  T *X = pool + off + BQ_X * L.np;
+  int count = symmetric ? 1 : 2, rb = 0;
+  if (zero) {
+    count++;
+    if ((count / 2) > max_iter) {
+      if (P.p[0].ip >= 0) X[P.p[0].ip] = T(0);
+      if (P.p[1].ip >= 0) X[P.p[1].ip] = T(0);
+      b_sync<WAVE>();
+      if (!symmetric) return;
+    }
+    b_half(P.p[1], pool, X, 1);
+    b_sync<WAVE>();
+    rb = 1;
+  }
+  for (; (count / 2) <= max_iter; count++) {
+    if (rb) b_half(P.p[0], pool, X, 0);
+    else b_half(P.p[1], pool, X, 0);
+    b_sync<WAVE>();
+    rb = !rb;
+  }
+}
+
+// way down: b of level l from the residual of the level above (not for the
+// top), its sweeps, its residual
+template <typename T, bool WAVE>
+__device__ __forceinline__ void b_down(T *pool, const BLevel<T> *__restrict__ lv, int l, int lc,
+                                       int nl, int pre, int symmetric)
+{
+  const BLevel<T> &L = lv[l];
+  const int off = LDS_ALIGN / (int)sizeof(T) + 9 * (int)(L.cum - lv[lc].cum);
+  // one pair a thread; threads without one work on pair 0 and store nothing
+  const int q = (int)threadIdx.x < L.npair ? (int)threadIdx.x : 0;
+  const bool act = (int)threadIdx.x < L.npair;
+  int m, j;
+  const int k = b_div(b_div(q, L.ncol, L.mcol, m), L.n[1], L.mrow, j);
+  if (l > lc) {
+    // restrict_point, for the pair's points
+    const BLevel<T> &F = lv[l - 1];
+    const int foff = LDS_ALIGN / (int)sizeof(T) + 9 * (int)(F.cum - lv[lc].cum), fnp = F.np;
+    const int d = F.dir, sd = d == 0 ? 1 : d == 1 ? F.s1 : F.s2, nd = F.n[d];
+    const int f0 = d == 0 ? 2 : 1, f1 = d == 1 ? 2 * F.s1 : F.s1, f2 = d == 2 ? 2 * F.s2 : F.s2;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const int i = 2 * m + c;
+      const bool in = i < L.n[0];
+      const int f = 2 * (d == 0 ? i : d == 1 ? j : k);
+      const int at = foff + (in ? i : 0) * f0 + j * f1 + k * f2;
+      const bool hl = in && f > 0, hh = in && f + 1 < nd;
+      const T lo = pool[hl ? at + BQ_P2 * fnp - sd : 0] * pool[hl ? at + BQ_T * fnp - sd : 0];
+      const T hi = pool[hh ? at + BQ_P1 * fnp + sd : 0] * pool[hh ? at + BQ_T * fnp + sd : 0];
+      const T rl = hl ? lo : T(0), rh = hh ? hi : T(0);
+      const T v = pool[at + BQ_T * fnp] + (rl + rh);
+      if (in && act) pool[off + BQ_B * L.np + i + j * L.s1 + k * L.s2] = v;
+    }
+  }
+  // the pair's own values of b are read back by the thread that stored them
+  BPair<T> P;
+  b_pair(P, (const T *)pool, L, off, m, j, k);
+  if (!act) P.p[0].ip = P.p[1].ip = -1;
+  if (l == nl - 1) {
+    b_sweeps<T, WAVE>(pool, L, off, P, 1, 1, symmetric);
+    return;
+  }
+  b_sweeps<T, WAVE>(pool, L, off, P, 1, pre, symmetric);
+  const T *X = pool + off + BQ_X * L.np;
+  T *R = pool + off + BQ_T * L.np;
+  b_resid(P.p[0], (const T *)pool, X, R);
+  b_resid(P.p[1], (const T *)pool, X, R);
+  b_sync<WAVE>();
+}
+
+// way up: x of level l corrected from the level below, and its sweeps
+template <typename T, bool WAVE>
+__device__ __forceinline__ void b_up(T *pool, const BLevel<T> *__restrict__ lv, int l, int lc,
+                                     int post, int symmetric)
+{
+  const BLevel<T> &L = lv[l], &G = lv[l + 1];
+  const int off = LDS_ALIGN / (int)sizeof(T) + 9 * (int)(L.cum - lv[lc].cum), np = L.np;
+  const int ex = LDS_ALIGN / (int)sizeof(T) + 9 * (int)(G.cum - lv[lc].cum) + BQ_X * G.np;
+  const int d = L.dir, nd = L.n[d], sc = d == 0 ? 1 : d == 1 ? G.s1 : G.s2;
+  const int q = (int)threadIdx.x < L.npair ? (int)threadIdx.x : 0;
+  const bool act = (int)threadIdx.x < L.npair;
+  int m, j;
+  const int k = b_div(b_div(q, L.ncol, L.mcol, m), L.n[1], L.mrow, j);
+  // prolong_point, for the pair's points
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    const int i = 2 * m + c;
+    const bool in = i < L.n[0];
+    const int f = d == 0 ? i : d == 1 ? j : k;
+    const int ip = off + (in ? i : 0) + j * L.s1 + k * L.s2;
+    const int ic = ex + (d == 0 ? (in ? i : 0) >> 1 : in ? i : 0) + (d == 1 ? j >> 1 : j) * G.s1 +
+                   (d == 2 ? k >> 1 : k) * G.s2;
+    const bool odd = (f & 1) != 0, hh = odd && f + 1 < nd;
+    const T e0 = pool[ic], e1 = pool[hh ? ic + sc : 0];
+    const T w1 = pool[ip + BQ_P1 * np], w2 = pool[ip + BQ_P2 * np], x = pool[ip + BQ_X * np];
+    T hi = T(0);
+    if (hh) hi = w2 * e1;
+    const T corr = b_fma(w1, e0, hi);
+    if (in && act) pool[ip + BQ_X * np] = x + (odd ? corr : e0);
+  }
+  BPair<T> P;
+  b_pair(P, (const T *)pool, L, off, m, j, k);
+  if (!act) P.p[0].ip = P.p[1].ip = -1;
+  b_sync<WAVE>();
+  b_sweeps<T, WAVE>(pool, L, off, P, 0, post, symmetric);
+}
+
+// element of a global array whose address comes from memory
+template <typename T> __device__ __forceinline__ T b_global(const T *p, long i)
+{
+  return *(const __attribute__((address_space(1))) T *)(p + i);
 }
 
 // bin / xout (the ensemble's levels 0 .. L-1 in one workgroup): the top
 // level's b comes from the FP64 vector bin and its x goes to xout, both in
 // the top level's ghosted layout; otherwise b and x are the top level's own
 template <typename T>
-__device__ void vcycle_lds(const LevelDev<T> *__restrict__ lev, int lc, int L, int pre,
-                           int post, int symmetric, const double *__restrict__ bin,
-                           double *__restrict__ xout)
+__device__ __forceinline__ void vcycle_lds(const BLevel<T> *__restrict__ lv, T *xtop, int lc,
+                                           int nl, int pre, int post, int symmetric,
+                                           const double *__restrict__ bin,
+                                           double *__restrict__ xout)
 {
   extern __shared__ __align__(LDS_ALIGN) unsigned char smem[];
-  const int nl = L - lc;
-  LevelDev<T> *lv = (LevelDev<T> *)smem;
-  T *pool = (T *)(smem + lds_level_table_bytes(nl, (long)sizeof(LevelDev<T>)));
-  if (threadIdx.x == 0) {
-    T *q = pool;
-    for (int m = 0; m < nl; m++) {
-      const LevelDev<T> &G = lev[lc + m];
-      LevelDev<T> D;
-      D.g = G.g;
-      D.g.s[0] = 1;
-      D.g.s[1] = G.g.n[0];
-      D.g.s[2] = G.g.n[0] * G.g.n[1];
-      D.dir = G.dir; D.o1 = G.o1; D.o2 = G.o2;
-      const long np = (long)G.g.n[0] * G.g.n[1] * G.g.n[2];
-      const long sh = 1 + D.g.s[1] + D.g.s[2];   // LIDX of (0, 0, 0)
-      D.A.c = q - sh; q += np;
-      for (int d = 0; d < 3; d++) { D.A.u[d] = q - sh; q += np; D.A.l[d] = nullptr; }
-      D.x = q - sh; q += np;
-      D.b = q - sh; q += np;
-      D.t = q - sh; q += np;
-      D.p1 = q - sh; q += np;
-      D.p2 = q - sh; q += np;
-      lv[m] = D;
+  T *pool = (T *)smem;
+  const int tid = threadIdx.x;
+  int nw = nl;                                  // first level of one wavefront
+  while (nw > lc && lv[nw - 1].npair <= 64) nw--;
+  if (tid == 0) pool[0] = T(0);
+  // copy in: the levels' pairs in chunks of 64, one wavefront each, CU chunks
+  // of loads in flight
+  constexpr int CU = 3;
+  int chunks = 0;
+  for (int l = lc; l < nl; l++) chunks += (lv[l].npair + 63) >> 6;
+  for (int c0 = __builtin_amdgcn_readfirstlane(tid >> 6); c0 < chunks; c0 += CU * (CWG / 64)) {
+    T v[CU][7][2];
+    int at[CU], np[CU];
+    bool in[CU], two[CU], top[CU];
+#pragma unroll
+    for (int u = 0; u < CU; u++) {
+      int c = c0 + u * (CWG / 64), l = lc;
+      const bool any = c < chunks;
+      c = any ? c : 0;
+      while (c >= (lv[l].npair + 63) >> 6) { c -= (lv[l].npair + 63) >> 6; l++; }
+      const BLevel<T> &D = lv[l];
+      const int q = 64 * c + (tid & 63);
+      in[u] = any && q < D.npair;
+      int m, j;
+      const int k = b_div(b_div(in[u] ? q : 0, D.ncol, D.mcol, m), D.n[1], D.mrow, j);
+      const int i = 2 * m;
+      two[u] = i + 1 < D.n[0];
+      top[u] = l == lc;
+      np[u] = D.np;
+      at[u] = LDS_ALIGN / (int)sizeof(T) + 9 * (int)(D.cum - lv[lc].cum) + i + j * D.s1 + k * D.s2;
+      const int ig = (i + 1) + (j + 1) * D.gs1 + (k + 1) * D.gs2, ih = ig + (two[u] ? 1 : 0);
+      const bool tr = l + 1 < nl;
+#pragma unroll
+      for (int a = 0; a < 6; a++) {
+        v[u][a][0] = (a < 4 || tr) ? b_global(D.g[a], ig) : T(0);
+        v[u][a][1] = (a < 4 || tr) ? b_global(D.g[a], ih) : T(0);
+      }
+      v[u][6][0] = !top[u] ? T(0) : bin ? (T)b_global(bin, ig) : b_global(D.gb, ig);
+      v[u][6][1] = !top[u] ? T(0) : bin ? (T)b_global(bin, ih) : b_global(D.gb, ih);
+    }
+#pragma unroll
+    for (int u = 0; u < CU; u++) {
+      if (!in[u]) continue;
+#pragma unroll
+      for (int a = 0; a < 6; a++) {
+        pool[at[u] + a * np[u]] = v[u][a][0];
+        if (two[u]) pool[at[u] + a * np[u] + 1] = v[u][a][1];
+      }
+      if (top[u]) {
+        pool[at[u] + BQ_B * np[u]] = v[u][6][0];
+        if (two[u]) pool[at[u] + BQ_B * np[u] + 1] = v[u][6][1];
+      }
     }
   }
   __syncthreads();
-  for (int m = 0; m < nl; m++) {
-    const LevelDev<T> &G = lev[lc + m];
-    const LevelDev<T> &D = lv[m];
-    const bool top = (m == 0);
-    const bool last = (m == nl - 1);
-    const int np = G.g.n[0] * G.g.n[1] * G.g.n[2];
-    for (int idx = threadIdx.x; idx < np; idx += blockDim.x) {
-      int i, j, k;
-      unflat(G.g, idx, i, j, k);
-      const long ig = LIDX(G.g, i, j, k);
-      const long il = LIDX(D.g, i, j, k);
-      D.A.c[il] = G.A.c[ig];
-      D.A.u[0][il] = G.A.u[0][ig];
-      D.A.u[1][il] = G.A.u[1][ig];
-      D.A.u[2][il] = G.A.u[2][ig];
-      if (!last) { D.p1[il] = G.p1[ig]; D.p2[il] = G.p2[ig]; }
-      if (top) D.b[il] = bin ? (T)bin[ig] : G.b[ig];
-    }
+  for (int l = lc; l < nw; l++) b_down<T, false>(pool, lv, l, lc, nl, pre, symmetric);
+  if (tid < 64) {
+    for (int l = nw; l < nl; l++) b_down<T, true>(pool, lv, l, lc, nl, pre, symmetric);
+    for (int l = nl - 2; l >= nw; l--) b_up<T, true>(pool, lv, l, lc, post, symmetric);
   }
   __syncthreads();
-  vcycle_block<T, false>(lv, 0, nl, pre, post, symmetric);
-  const LevelDev<T> &G = lev[lc];
-  const LevelDev<T> &D = lv[0];
-  if (xout) {
-    FOR_POINTS(G.g, xout[LIDX(G.g, i, j, k)] = (double)D.x[LIDX(D.g, i, j, k)]);
-  } else {
-    FOR_POINTS(G.g, G.x[LIDX(G.g, i, j, k)] = D.x[LIDX(D.g, i, j, k)]);
+  for (int l = min(nw - 1, nl - 2); l >= lc; l--) b_up<T, false>(pool, lv, l, lc, post, symmetric);
+  const BLevel<T> &D = lv[lc];
+  const int off = LDS_ALIGN / (int)sizeof(T) + BQ_X * D.np;
+  for (int q = tid; q < D.npair; q += CWG) {
+    int m, j;
+    const int k = b_div(b_div(q, D.ncol, D.mcol, m), D.n[1], D.mrow, j);
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const int i = 2 * m + c;
+      if (i >= D.n[0]) continue;
+      const int ig = (i + 1) + (j + 1) * D.gs1 + (k + 1) * D.gs2;
+      const T v = pool[off + i + j * D.s1 + k * D.s2];
+      if (xout) stg_o(xout, (unsigned)ig, (double)v);
+      else stg_o(xtop, (unsigned)ig, v);
+    }
   }
 }
 
 template <typename T>
-__global__ __launch_bounds__(CWG) void k_coarse_vcycle_lds(const LevelDev<T> *__restrict__ lev,
-                                                           int lc, int L, int pre, int post,
-                                                           int symmetric)
+__global__ __launch_bounds__(CWG) void k_coarse_vcycle_lds(const BLevel<T> *__restrict__ lv,
+                                                           T *xtop, int lc, int L, int pre,
+                                                           int post, int symmetric)
 {
-  vcycle_lds<T>(lev, lc, L, pre, post, symmetric, nullptr, nullptr);
+  vcycle_lds<T>(lv, xtop, lc, L, pre, post, symmetric, nullptr, nullptr);
 }
 
+// pairs of x-neighbours of a level: the LDS bottom has one per thread
+static long lds_pairs(const int *n) { return (long)((n[0] + 1) / 2) * n[1] * n[2]; }
+
 // LDS bytes of the bottom levels lc .. L-1 in k_coarse_vcycle_lds
-static long lds_bottom_bytes(const int (*n)[3], int lc, int L, size_t es, size_t rec)
+static long lds_bottom_bytes(const int (*n)[3], int lc, int L, size_t es)
 {
-  long b = lds_level_table_bytes(L - lc, (long)rec);
+  long b = LDS_ALIGN;                            // the zero word
   for (int l = lc; l < L; l++) b += 9L * (long)es * n[l][0] * n[l][1] * n[l][2];
   return b;
 }
@@ -1661,6 +1929,7 @@ struct pfhip_mg {
   long dqp_n;                  // partials per sum that dqp holds
   int tuned;                   // pv chosen (at the first V-cycle)
   void *levdev;                // device LevelDev<T>[L]
+  void *bldev;                 // device BLevel<T>[L]
   long lds_bytes;              // > 0: the bottom runs in LDS (k_coarse_vcycle_lds)
   int use_graph;               // replay the captured V-cycle (mg_capture)
   hipStream_t cs;              // capture stream
@@ -1705,6 +1974,31 @@ template <typename T> static int upload_levels(pfhip_mg *mg)
   int rc = pfhip_malloc(&mg->levdev, (long)sizeof(LevelDev<T>) * mg->L);
   if (rc) return rc;
   HIPCHK(hipMemcpy(mg->levdev, h, sizeof(LevelDev<T>) * mg->L, hipMemcpyHostToDevice));
+  BLevel<T> bl[MAXL];
+  memset(bl, 0, sizeof(bl));
+  long cum = 0;
+  for (int l = 0; l < mg->L; l++) {
+    BLevel<T> &D = bl[l];
+    const int *n = mg->n[l];
+    for (int q = 0; q < 3; q++) D.n[q] = n[q];
+    D.dir = h[l].dir;
+    D.s1 = n[0]; D.s2 = n[0] * n[1];
+    D.gs1 = h[l].g.s[1]; D.gs2 = h[l].g.s[2];
+    D.cum = (unsigned)cum;
+    D.np = (int)npts(n);
+    cum += D.np;
+    D.ncol = (n[0] + 1) >> 1;
+    D.npair = D.ncol * n[1] * n[2];
+    D.mcol = D.ncol > 1 ? (unsigned)((0x100000000ULL + D.ncol - 1) / D.ncol) : 0;
+    D.mrow = n[1] > 1 ? (unsigned)((0x100000000ULL + n[1] - 1) / n[1]) : 0;
+    D.g[0] = h[l].A.c;
+    for (int q = 0; q < 3; q++) D.g[1 + q] = h[l].A.u[q];
+    D.g[4] = h[l].p1; D.g[5] = h[l].p2;
+    D.gb = h[l].b;
+  }
+  rc = pfhip_malloc(&mg->bldev, (long)sizeof(BLevel<T>) * mg->L);
+  if (rc) return rc;
+  HIPCHK(hipMemcpy(mg->bldev, bl, sizeof(BLevel<T>) * mg->L, hipMemcpyHostToDevice));
   return PFHIP_OK;
 }
 
@@ -1772,10 +2066,9 @@ static int mg_create(pfhip_problem *pb, int max_levels, int pre, int post, int s
           hipSuccess)
     lds_max = 0;
   if (!full && lds_budget > 0 && lds_budget <= lds_max && !(env && *env)) {
-    const size_t rec = (precision == 64) ? sizeof(LevelDev<double>) : sizeof(LevelDev<float>);
     for (l = 1; l <= mg->L - 2; l++) {
-      const long bytes = lds_bottom_bytes(mg->n, l, mg->L, es, rec);
-      if (bytes <= lds_budget && npts(mg->n[l]) <= small) {
+      const long bytes = lds_bottom_bytes(mg->n, l, mg->L, es);
+      if (bytes <= lds_budget && npts(mg->n[l]) <= small && lds_pairs(mg->n[l]) <= CWG) {
         mg->lc = l;
         mg->lds_bytes = bytes;
         break;
@@ -1851,6 +2144,7 @@ extern "C" int pfhip_mg_destroy(pfhip_mg *mg)
     for (int q = 0; q < 13; q++) if (mg->raw[l][q]) hipFree(mg->raw[l][q]);
   }
   if (mg->levdev) hipFree(mg->levdev);
+  if (mg->bldev) hipFree(mg->bldev);
   free(mg);
   return PFHIP_OK;
 }
@@ -2278,7 +2572,7 @@ static int mg_apply_seq(pfhip_mg *mg, const double *bin, double *xout, hipStream
   // level's solve is RedBlackGSPoint with MaxIter 1
   if (lc <= L - 2 && mg->lds_bytes > 0) {
     hipLaunchKernelGGL(k_coarse_vcycle_lds<T>, dim3(1), dim3(CWG), (unsigned)mg->lds_bytes, st,
-                       (const LevelDev<T> *)mg->levdev, lc, L, mg->pre, mg->post,
+                       (const BLevel<T> *)mg->bldev, (T *)mg->x[lc], lc, L, mg->pre, mg->post,
                        mg->symmetric);
     LAUNCHCHK();
   } else if (lc <= L - 2) {
@@ -2489,6 +2783,7 @@ struct EnsLSeg { int m, blk0; };
 
 template <typename T> struct EnsLv {
   const LevelDev<T> *lev;
+  const BLevel<T> *bl;
   const double *bin;    // this round's V-cycle right-hand side (FP64)
   double *xout;         // and result
   int L, lc, pre, post, symmetric, act;
@@ -2611,7 +2906,7 @@ __global__ __launch_bounds__(CWG) void k_ens_vcycle_lds(const EnsLv<T> *__restri
 {
   const EnsLv<T> &mm = M[list[blockIdx.x]];
   if (!mm.act) return;                          // uniform over the workgroup
-  vcycle_lds<T>(mm.lev, mm.lc, mm.L, mm.pre, mm.post, mm.symmetric,
+  vcycle_lds<T>(mm.bl, mm.lev[mm.lc].x, mm.lc, mm.L, mm.pre, mm.post, mm.symmetric,
                 mm.lc == 0 ? mm.bin : nullptr, mm.lc == 0 ? mm.xout : nullptr);
 }
 
@@ -2690,7 +2985,6 @@ extern "C" int pfhip_ens_mg_plan_create(pfhip_mg *const *mgs, int n, pfhip_ens_m
     lds_max = 0;
   const bool lds = !(se && *se) && lds_budget > 0 && lds_budget <= lds_max;
   const size_t es = (p->prec == 64) ? sizeof(double) : sizeof(float);
-  const size_t rec = (p->prec == 64) ? sizeof(LevelDev<double>) : sizeof(LevelDev<float>);
   for (int m = 0; m < n; m++) {
     const pfhip_mg *mg = mgs[m];
     if (mg->prec != p->prec || mg->full || mg->pre != p->pre || mg->post != p->post ||
@@ -2702,8 +2996,8 @@ extern "C" int pfhip_ens_mg_plan_create(pfhip_mg *const *mgs, int n, pfhip_ens_m
     int lc = mg->L - 1;
     if (lds) {
       for (int l = 0; l < mg->L; l++) {
-        const long b = lds_bottom_bytes(mg->n, l, mg->L, es, rec);
-        if (b <= lds_budget) {
+        const long b = lds_bottom_bytes(mg->n, l, mg->L, es);
+        if (b <= lds_budget && lds_pairs(mg->n[l]) <= CWG) {
           lc = l;
           if (b > p->lds_bytes) p->lds_bytes = b;
           break;
@@ -2889,6 +3183,7 @@ static int ens_mg_launch(pfhip_ens_mgplan *p, pfhip_ens_req *const *rq, int n, i
     }
     EnsLv<T> &e = M[m];
     e.lev = (const LevelDev<T> *)mg->levdev;
+    e.bl = (const BLevel<T> *)mg->bldev;
     e.bin = rq[r]->x;
     e.xout = rq[r]->z;
     e.L = mg->L; e.lc = p->lc[m];

@@ -115,3 +115,27 @@ def test_residual_and_jacobian_plane_chunks(gpu, shape):
         scale = np.max(np.abs(I(B[0])))
         for q in ((0, 2, 4, 6) if symm else range(7)):
             assert np.max(np.abs(I(A[q]) - I(B[q]))) <= 1e-11 * scale, (symm, q)
+
+
+@pytest.mark.parametrize("shape", [(2, 1, 1), (1, 1, 9), (3, 5, 7), (16, 9, 14), (1, 64, 64), (33, 8, 8)])
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("sweeps", [(1, 1, 1), (1, 1, 0), (2, 2, 0), (0, 1, 0), (2, 0, 1)])
+def test_multigrid_bottom_levels(gpu, shape, precision, sweeps):
+    """V-cycles whose levels all run in the one-workgroup bottom but the
+    first: single points, odd extents, one point per row (more pairs than
+    threads keep a level on the grid), against the oracle."""
+    api = _api()
+    pre, post, sym = sweeps
+    prob = cases.hetero(*shape, seed=21)
+    gp = api.GPUProblem(prob)
+    A = cases.full_operator(prob, 22, symmetric=True)
+    b = np.zeros(prob.shape)
+    prob.interior(b)[...] = np.random.default_rng(23).normal(size=prob.interior(b).shape)
+    mg = api.GPUMultigrid(gp, pre, post, sym, precision=precision)
+    mg.setup(A)
+    got = prob.interior(mg.apply(b))
+    om = O.MG(prob, pre, post, sym)
+    om.setup(A)
+    want = prob.interior(om.apply(b))
+    tol = 1e-11 if precision == 64 else 2e-5
+    assert np.max(np.abs(got - want)) <= tol * np.max(np.abs(want))
