@@ -46,6 +46,13 @@
 #define MG_LDS_DEFAULT (144L * 1024)   // LDS of the bottom-of-cycle workgroup
 #define CWG 1024
 #define MAX_SWEEPS 64
+#ifndef BLOCK_POINTS
+#define BLOCK_POINTS 300000L
+#endif
+#ifndef BLOCK_RATE
+#define BLOCK_RATE 50000.0
+#endif
+#define BLOCK_SWEEPS 4
 
 struct LGeom {
   int n[3];
@@ -1900,7 +1907,204 @@ __global__ __launch_bounds__(CWG) void k_coarse_setup(const LevelDev<T> *__restr
   }
 }
 
+// ---- all of a level's work on one block, in one launch ------------------------
+// The levels between the marching kernels' and the one-workgroup bottom are
+// too small for either: a half-sweep, a transfer or a pair takes 4 to 10 us
+// whatever it does, six of them a level.  Here a workgroup owns a block of
+// points, reads it with a rim of neighbours wide enough for everything that
+// follows, and does the whole visit in LDS: on the way down the sweeps from a
+// zero guess, the residual and its restriction; on the way up the correction
+// and the sweeps.  The rim's points are recomputed by the blocks that share
+// them (each half-sweep makes one layer of it stale).  A thread keeps the
+// rows of one or two x pairs in registers; x alone goes through LDS.  Point by
+// point the operations and their order are the separate kernels'.
+template <typename T> struct LBlock {
+  LGeom g, gc;
+  Mat<T> A;
+  int d;                       // coarsening direction
+  int o[3], e[3], hl[3], t[3]; // owned points, points read, rim below, blocks
+  unsigned mcol, mrow;         // b_div multipliers of e[0] / 2 and e[1]
+  int nh;                      // half-sweeps, red first
+  const T *b, *xin, *ec, *p1, *p2;
+  T *xout, *bc;
+  // level 0: the solver's FP64 vectors (din is converted into bout as well);
+  // with io their addresses and din's factor come from there
+  const double *din;
+  double *dout, dsc;
+  T *bout;
+  void *const *io;
+};
+enum { LB_ZERO = 0, LB_PROLONG = 1 };
+
+// a block's points: PP pairs per thread; SRC: what x starts from; with
+// LB_ZERO the residual is restricted into bc at the end
+template <typename T, int PP, int SRC>
+__device__ __forceinline__ void lvl_block(const LBlock<T> &B, int blk, T *X)
+{
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const int ex = B.e[0], ey = B.e[1], ez = B.e[2];
+  const int L1 = ex + 2, L2 = L1 * (ey + 2), nl = L2 * (ez + 2);
+  T *R = X + nl;
+  const int n0 = B.g.n[0], n1 = B.g.n[1], n2 = B.g.n[2];
+  const int bx = blk % B.t[0], br = blk / B.t[0];
+  const int o0 = bx * B.o[0], o1 = (br % B.t[1]) * B.o[1], o2 = (br / B.t[1]) * B.o[2];
+  const int e0 = max(o0 - B.hl[0], 0), e1 = max(o1 - B.hl[1], 0), e2 = max(o2 - B.hl[2], 0);
+  const int sy = B.g.s[1], sz = B.g.s[2];
+  const int ncol = ex >> 1, npair = ncol * ey * ez;
+  const double *din = B.din;
+  double *dout = B.dout;
+  double dsc = B.dsc;
+  if (B.io && din) { din = (const double *)B.io[0]; dsc = io_double(B.io, 2); }
+  if (B.io && dout) dout = (double *)B.io[1];
+  for (int q = tid; q < nl; q += nt) X[q] = T(0);
+  // rows of the thread's points, by colour: [1] red, [0] black
+  T c[PP][2], b[PP][2], aw[PP][2], ae[PP][2], as[PP][2], an[PP][2], al[PP][2], au[PP][2];
+  T x0[PP][2];
+  int lp[PP][2], gp[PP][2];    // place in X, and in global memory if owned
+  bool in[PP][2];
+#pragma unroll
+  for (int u = 0; u < PP; u++) {
+    const int q = tid + u * nt;
+    const bool act = q < npair;
+    int m, jl;
+    const int kl = b_div(b_div(act ? q : 0, ncol, B.mcol, m), ey, B.mrow, jl);
+    const int j = e1 + jl, k = e2 + kl;
+    const int odd = (e0 + j + k) & 1;
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+      const int cc = a ? odd ^ 1 : odd, i = e0 + 2 * m + cc;
+      const bool ok = act && i < n0 && j < n1 && k < n2;
+      const int ic = min(i, n0 - 1), jc = min(j, n1 - 1), kc = min(k, n2 - 1);
+      const int ip = (ic + 1) + (jc + 1) * sy + (kc + 1) * sz;
+      in[u][a] = ok;
+      lp[u][a] = (2 * m + cc + 1) + (jl + 1) * L1 + (kl + 1) * L2;
+      const bool own = ok && i >= o0 && i < o0 + B.o[0] && j >= o1 && j < o1 + B.o[1] &&
+                       k >= o2 && k < o2 + B.o[2];
+      gp[u][a] = own ? ip : -1;
+      // unconditional loads from clamped places
+      const T vc = B.A.c[ip], ve = B.A.u[0][ip], vn = B.A.u[1][ip], vu = B.A.u[2][ip];
+      const T vw = B.A.u[0][ip - 1], vs = B.A.u[1][ip - sy], vl = B.A.u[2][ip - sz];
+      const T vb = din ? (T)(dsc * ldg_o(din, (unsigned)ip)) : B.b[ip];
+      c[u][a] = ok ? vc : T(1);
+      b[u][a] = ok ? vb : T(0);
+      aw[u][a] = ok && ic > 0 ? vw : T(0);
+      ae[u][a] = ok && ic + 1 < n0 ? ve : T(0);
+      as[u][a] = ok && jc > 0 ? vs : T(0);
+      an[u][a] = ok && jc + 1 < n1 ? vn : T(0);
+      al[u][a] = ok && kc > 0 ? vl : T(0);
+      au[u][a] = ok && kc + 1 < n2 ? vu : T(0);
+      if (SRC == LB_PROLONG) {
+        // prolong_point
+        const int d = B.d, f = d == 0 ? ic : d == 1 ? jc : kc, nd = B.g.n[d];
+        const int cs = d == 0 ? 1 : B.gc.s[d];
+        const int ci = (d == 0 ? ic >> 1 : ic) + 1 + ((d == 1 ? jc >> 1 : jc) + 1) * B.gc.s[1] +
+                       ((d == 2 ? kc >> 1 : kc) + 1) * B.gc.s[2];
+        const bool of = (f & 1) != 0, hh = of && f + 1 < nd;
+        const T g0 = B.ec[ci], g1 = B.ec[hh ? ci + cs : ci];
+        const T w1 = B.p1[ip], w2 = B.p2[ip], xv = B.xin[ip];
+        T hi = T(0);
+        if (hh) hi = w2 * g1;
+        const T corr = b_fma(w1, g0, hi);
+        x0[u][a] = ok ? xv + (of ? corr : g0) : T(0);
+      }
+    }
+  }
+  __syncthreads();             // X is zero
+  if (SRC == LB_PROLONG) {
+#pragma unroll
+    for (int u = 0; u < PP; u++)
+#pragma unroll
+      for (int a = 0; a < 2; a++)
+        if (in[u][a]) X[lp[u][a]] = x0[u][a];
+    lds_barrier();
+  } else if (din) {
+#pragma unroll
+    for (int u = 0; u < PP; u++)
+#pragma unroll
+      for (int a = 0; a < 2; a++)
+        if (gp[u][a] >= 0) B.bout[gp[u][a]] = b[u][a];
+  }
+  for (int h = 0; h < B.nh; h++) {
+#pragma unroll
+    for (int u = 0; u < PP; u++) {
+#pragma clang fp contract(off)
+      const bool red = (h & 1) == 0;
+      // the colour's row (selects, not an indexed register array)
+      const T vc = red ? c[u][1] : c[u][0], vb = red ? b[u][1] : b[u][0];
+      const int p = red ? lp[u][1] : lp[u][0];
+      const bool ok = red ? in[u][1] : in[u][0];
+      T v;
+      if (SRC == LB_ZERO && h == 0) {
+        v = gs_div(vb, vc);
+      } else {
+        const T w = (red ? aw[u][1] : aw[u][0]) * X[p - 1];
+        const T e = (red ? ae[u][1] : ae[u][0]) * X[p + 1];
+        const T so = (red ? as[u][1] : as[u][0]) * X[p - L1];
+        const T no = (red ? an[u][1] : an[u][0]) * X[p + L1];
+        const T lo = (red ? al[u][1] : al[u][0]) * X[p - L2];
+        const T up = (red ? au[u][1] : au[u][0]) * X[p + L2];
+        const T sum = w + e + so + no + lo + up;
+        v = gs_div(vb - sum, vc);
+      }
+      if (ok) X[p] = v;
+    }
+    lds_barrier();
+  }
+#pragma unroll
+  for (int u = 0; u < PP; u++) {
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+      const int p = lp[u][a];
+      const T xv = X[p];
+      if (gp[u][a] >= 0) {
+        if (dout) stg_o(dout, (unsigned)gp[u][a], (double)xv);
+        else B.xout[gp[u][a]] = xv;
+      }
+      if (SRC == LB_ZERO) {
+        T v = c[u][a] * xv;
+        v = b_fma(aw[u][a], X[p - 1], v);
+        v = b_fma(ae[u][a], X[p + 1], v);
+        v = b_fma(as[u][a], X[p - L1], v);
+        v = b_fma(an[u][a], X[p + L1], v);
+        v = b_fma(al[u][a], X[p - L2], v);
+        v = b_fma(au[u][a], X[p + L2], v);
+        if (in[u][a]) R[p] = b[u][a] - v;
+      }
+    }
+  }
+  if (SRC != LB_ZERO) return;
+  lds_barrier();
+  // restrict_point for the block's coarse points
+  const int d = B.d, nd = B.g.n[d];
+  const int w0 = d == 0 ? B.o[0] >> 1 : B.o[0], w1 = d == 1 ? B.o[1] >> 1 : B.o[1];
+  const int w2 = d == 2 ? B.o[2] >> 1 : B.o[2];
+  const int gd = d == 0 ? 1 : B.g.s[d], ld = d == 0 ? 1 : d == 1 ? L1 : L2;
+  for (int q = tid; q < w0 * w1 * w2; q += nt) {
+    const int i = (d == 0 ? o0 >> 1 : o0) + q % w0, r = q / w0;
+    const int j = (d == 1 ? o1 >> 1 : o1) + r % w1, k = (d == 2 ? o2 >> 1 : o2) + r / w1;
+    if (i >= B.gc.n[0] || j >= B.gc.n[1] || k >= B.gc.n[2]) continue;
+    const int fi = d == 0 ? 2 * i : i, fj = d == 1 ? 2 * j : j, fk = d == 2 ? 2 * k : k;
+    const int f = d == 0 ? fi : d == 1 ? fj : fk;
+    const int ip = (fi + 1) + (fj + 1) * sy + (fk + 1) * sz;
+    const int p = (fi - e0 + 1) + (fj - e1 + 1) * L1 + (fk - e2 + 1) * L2;
+    const bool hl = f > 0, hh = f + 1 < nd;
+    const T c2 = B.p2[hl ? ip - gd : ip], c1 = B.p1[hh ? ip + gd : ip];
+    const T pl = c2 * R[hl ? p - ld : p], ph = c1 * R[hh ? p + ld : p];
+    const T lo = hl ? pl : T(0), hi = hh ? ph : T(0);
+    B.bc[(i + 1) + (j + 1) * B.gc.s[1] + (k + 1) * B.gc.s[2]] = R[p] + (lo + hi);
+  }
+}
+
+template <typename T, int PP, int SRC>
+__global__ __launch_bounds__(CWG) void k_lvl_block(LBlock<T> B)
+{
+  extern __shared__ __align__(LDS_ALIGN) unsigned char smem[];
+  lvl_block<T, PP, SRC>(B, blockIdx.x, (T *)smem);
+}
+
 // ---- host side ----------------------------------------------------------------
+// a level's block shape: owned points, points read and rim below, per axis
+struct LvlShape { int o[3], e[3], hl[3], t[3], pp; long blocks; };
 struct pfhip_mg {
   pfhip_problem *pb;
   int L, prec, pre, post, symmetric;
@@ -1928,6 +2132,9 @@ struct pfhip_mg {
   double *dqp;                 // their per-workgroup partials
   long dqp_n;                  // partials per sum that dqp holds
   int tuned;                   // pv chosen (at the first V-cycle)
+  int blk[MAXL];               // the level's visits run as block launches (k_lvl_block)
+  LvlShape down[MAXL], up[MAXL];
+  void *xres[MAXL];            // a V-cycle's result on each level (set per call)
   void *levdev;                // device LevelDev<T>[L]
   void *bldev;                 // device BLevel<T>[L]
   long lds_bytes;              // > 0: the bottom runs in LDS (k_coarse_vcycle_lds)
@@ -1939,6 +2146,7 @@ struct pfhip_mg {
 
 template <typename T> static int tune_pairs(pfhip_mg *mg, hipStream_t st);
 static int rbgs_forced();
+static void plan_blocks(pfhip_mg *mg);
 
 template <typename T> static Mat<T> matof(pfhip_mg *mg, int l)
 {
@@ -2111,6 +2319,7 @@ static int mg_create(pfhip_problem *pb, int max_levels, int pre, int post, int s
     rc = (precision == 64) ? upload_levels<double>(mg) : upload_levels<float>(mg);
   if (rc != PFHIP_OK) { pfhip_mg_destroy(mg); return rc; }
   int forced = rbgs_forced();
+  plan_blocks(mg);
   for (l = 0; l < MAXL; l++) mg->pv[l] = (forced >= 0) ? forced : 0;
   mg->pv_din = mg->pv_dout = (forced >= 0) ? forced : 0;
   mg->tuned = (forced >= 0) || !mg->fuse || full;
@@ -2257,6 +2466,136 @@ static int sweep_list(int symmetric, int zero, int max_iter, HalfSweep *seq, int
   return n;
 }
 
+// The block shape of a level of extents n: the owned extents (even along d)
+// whose rim is the smallest work, among those that a workgroup of CWG threads
+// holds with pp pairs each.  hl, hh: rim below and above, per axis.
+static bool block_shape(const int *n, int d, const int *hl, const int *hh, size_t es,
+                        LvlShape *best)
+{
+  static const int sizes[] = { 2, 4, 6, 8, 12, 16, 24, 28, 32, 48, 56 };
+  const int ns = (int)(sizeof(sizes) / sizeof(sizes[0]));
+  double cost = 0.0;
+  bool found = false;
+  for (int a = 0; a <= ns; a++)
+    for (int b = 0; b <= ns; b++)
+      for (int c = 0; c <= ns; c++) {
+        const int pick[3] = { a, b, c };
+        LvlShape S;
+        long pts = 1, blocks = 1;
+        bool ok = true;
+        for (int q = 0; q < 3; q++) {
+          // the last choice is the whole extent (rounded up to even along d)
+          const int whole = q == d ? (n[q] + 1) & ~1 : n[q];
+          S.o[q] = pick[q] == ns ? whole : sizes[pick[q]];
+          ok = ok && S.o[q] <= whole;
+          S.hl[q] = S.o[q] >= n[q] ? 0 : hl[q];
+          S.e[q] = S.o[q] >= n[q] ? n[q] : S.o[q] + hl[q] + hh[q];
+          if (S.e[q] > n[q]) S.e[q] = n[q];
+          if (q == 0) S.e[q] = (S.e[q] + 1) & ~1;
+          S.t[q] = (n[q] + S.o[q] - 1) / S.o[q];
+          pts *= S.e[q];
+          blocks *= S.t[q];
+        }
+        const long pairs = pts / 2;
+        const long lds = 2 * (long)es * (S.e[0] + 2) * (S.e[1] + 2) * (S.e[2] + 2);
+        if (!ok || pairs > 2 * CWG || lds > 65536) continue;
+        S.pp = pairs > CWG ? 2 : 1;
+        S.blocks = blocks;
+        // microseconds, fitted to measurements: a block's own latency, which
+        // grows with its wavefronts, and the chip's throughput
+        const double w = 4.0 + 2.5 * (double)pairs / CWG + (double)(blocks * pairs) / BLOCK_RATE;
+        if (!found || w < cost) { cost = w; *best = S; found = true; }
+      }
+  return found;
+}
+
+// Which levels run as block launches.  (rule: see k_lvl_block's measurements)
+static void plan_blocks(pfhip_mg *mg)
+{
+  const char *e = getenv("PFHIP_MG_BLOCK");
+  const long most = (e && *e) ? atol(e) : BLOCK_POINTS;
+  if (!mg->fuse || mg->full || rbgs_forced() >= 0) return;
+  HalfSweep seq[2 * MAX_SWEEPS + 4];
+  int fill;
+  const int nd = sweep_list(mg->symmetric, 1, mg->pre, seq, &fill);
+  if (fill || nd < 1) return;
+  const int nu = sweep_list(mg->symmetric, 0, mg->post, seq, &fill);
+  if (nu < 1 || nd > BLOCK_SWEEPS || nu > BLOCK_SWEEPS) return;
+  for (int l = 0; l < mg->lc; l++) {
+    if (npts(mg->n[l]) > most) continue;
+    const int d = mg->dir[l];
+    int hl[3], hh[3];
+    for (int q = 0; q < 3; q++) { hl[q] = nd + (q == d ? 1 : 0); hh[q] = nd; }
+    const size_t es = mg->prec == 64 ? sizeof(double) : sizeof(float);
+    if (!block_shape(mg->n[l], d, hl, hh, es, &mg->down[l])) continue;
+    for (int q = 0; q < 3; q++) hl[q] = hh[q] = nu;
+    if (!block_shape(mg->n[l], d, hl, hh, es, &mg->up[l])) continue;
+    mg->blk[l] = 1;
+  }
+}
+
+template <typename T>
+static LBlock<T> block_args(pfhip_mg *mg, int l, const LvlShape &S, int nh)
+{
+  LBlock<T> B;
+  memset(&B, 0, sizeof(B));
+  B.g = lgeom(mg->n[l]); B.gc = lgeom(mg->n[l + 1]);
+  B.A = matof<T>(mg, l);
+  B.d = mg->dir[l];
+  for (int q = 0; q < 3; q++) { B.o[q] = S.o[q]; B.e[q] = S.e[q]; B.hl[q] = S.hl[q]; B.t[q] = S.t[q]; }
+  const unsigned ncol = (unsigned)S.e[0] / 2, row = (unsigned)S.e[1];
+  B.mcol = ncol > 1 ? (unsigned)((0x100000000ULL + ncol - 1) / ncol) : 0;
+  B.mrow = row > 1 ? (unsigned)((0x100000000ULL + row - 1) / row) : 0;
+  B.nh = nh;
+  B.b = (const T *)mg->b[l];
+  B.p1 = (const T *)mg->p1[l]; B.p2 = (const T *)mg->p2[l];
+  B.dsc = 1.0;
+  return B;
+}
+
+template <typename T, int SRC>
+static void launch_block(const LBlock<T> &B, const LvlShape &S, hipStream_t st)
+{
+  const int pairs = S.e[0] / 2 * S.e[1] * S.e[2];
+  const int nt = ((pairs + S.pp - 1) / S.pp + 63) & ~63;
+  const unsigned lds = (unsigned)((SRC == LB_ZERO ? 2 : 1) * sizeof(T) * (S.e[0] + 2) *
+                                  (S.e[1] + 2) * (S.e[2] + 2));
+  if (S.pp == 2)
+    hipLaunchKernelGGL((k_lvl_block<T, 2, SRC>), dim3((unsigned)S.blocks), dim3(nt), lds, st, B);
+  else
+    hipLaunchKernelGGL((k_lvl_block<T, 1, SRC>), dim3((unsigned)S.blocks), dim3(nt), lds, st, B);
+}
+
+// the two visits of a level that plan_blocks chose; din / dout: level 0's
+// FP64 vectors
+template <typename T>
+static int block_down(pfhip_mg *mg, int l, const double *din, void *const *io, hipStream_t st)
+{
+  HalfSweep seq[2 * MAX_SWEEPS + 4];
+  int fill;
+  LBlock<T> B = block_args<T>(mg, l, mg->down[l], sweep_list(mg->symmetric, 1, mg->pre, seq, &fill));
+  B.xout = (T *)mg->x[l];
+  B.bc = (T *)mg->b[l + 1];
+  if (din) { B.din = din; B.dsc = mg->bscale; B.bout = (T *)mg->b[l]; B.io = io; }
+  launch_block<T, LB_ZERO>(B, mg->down[l], st);
+  LAUNCHCHK();
+  return PFHIP_OK;
+}
+template <typename T>
+static int block_up(pfhip_mg *mg, int l, double *dout, void *const *io, hipStream_t st)
+{
+  HalfSweep seq[2 * MAX_SWEEPS + 4];
+  int fill;
+  LBlock<T> B = block_args<T>(mg, l, mg->up[l], sweep_list(mg->symmetric, 0, mg->post, seq, &fill));
+  B.xin = (const T *)mg->x[l];
+  B.ec = (const T *)mg->xres[l + 1];
+  B.xout = (T *)mg->xa[l];
+  if (dout) { B.dout = dout; B.io = io; }
+  launch_block<T, LB_PROLONG>(B, mg->up[l], st);
+  LAUNCHCHK();
+  return PFHIP_OK;
+}
+
 // Fused pair tile shapes (rows TY of a tile, z-chunk KC).  Each multigrid
 // times them per grid level when it is created (tune_pairs) and keeps the
 // fastest; PFHIP_RBGS_VARIANT=v forces shape v on every level.
@@ -2382,7 +2721,7 @@ static int tune_pairs(pfhip_mg *mg, hipStream_t st, const double *bin, double *x
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   for (int l = 0; l < mg->lc; l++) {
-    if (!mg->xa[l]) continue;
+    if (!mg->xa[l] || mg->blk[l]) continue;
     LGeom g = lgeom(mg->n[l]);
     Mat<T> A = matof<T>(mg, l);
     const bool fp64_forms = l == 0 && bin && xout && (g.n[0] % 2) == 0;
@@ -2536,7 +2875,7 @@ static int mg_apply_seq(pfhip_mg *mg, const double *bin, double *xout, hipStream
   const int n0 = sweep_list(mg->symmetric, 1, mg->pre, seq0, &fill0);
   const bool din = mg->fuse && !mg->full && mg->xa[0] && (g0.n[0] % 2) == 0 && !fill0 &&
                    n0 >= 2 && seq0[0].par == 1 && seq0[0].init && seq0[1].par == 0;
-  if (!din) {
+  if (!din && !mg->blk[0]) {
     if (io)
       hipLaunchKernelGGL((k_convert_io<double, T>), dim3(ntiles(g0)), LBLOCK, 0, st, g0, bin,
                          (T *)mg->b[0], io, 0);
@@ -2547,6 +2886,10 @@ static int mg_apply_seq(pfhip_mg *mg, const double *bin, double *xout, hipStream
   }
   int l;
   for (l = 0; l < lc; l++) {
+    if (mg->blk[l]) {
+      if ((rc = block_down<T>(mg, l, l == 0 ? bin : nullptr, io, st))) return rc;
+      continue;
+    }
     if ((rc = rbgs<T>(mg, l, 1, mg->pre, st, nullptr, nullptr, (l == 0 && din) ? bin : nullptr,
                       io)))
       return rc;
@@ -2588,21 +2931,29 @@ static int mg_apply_seq(pfhip_mg *mg, const double *bin, double *xout, hipStream
   } else {
     if ((rc = rbgs<T>(mg, L - 1, 1, 1, st))) return rc;
   }
+  mg->xres[lc] = mg->x[lc];
   for (l = lc - 1; l >= 0; l--) {
     LGeom gf = lgeom(mg->n[l]), gc = lgeom(mg->n[l + 1]);
+    if (mg->blk[l]) {
+      if ((rc = block_up<T>(mg, l, l == 0 ? xout : nullptr, io, st))) return rc;
+      mg->xres[l] = mg->xa[l];
+      wrote = wrote || l == 0;
+      continue;
+    }
     if (mg->cz && mg->dir[l] == 2) {
       const unsigned nb = (unsigned)((gf.n[0] + 63) / 64) * ((gf.n[1] + 3) / 4);
       hipLaunchKernelGGL(k_prolong_z<T>, dim3((nb + 7u) & ~7u), LBLOCK, 0, st, gf, gc,
-                         (const T *)mg->x[l + 1], (T *)mg->x[l], (const T *)mg->p1[l],
+                         (const T *)mg->xres[l + 1], (T *)mg->x[l], (const T *)mg->p1[l],
                          (const T *)mg->p2[l]);
     } else {
       hipLaunchKernelGGL(k_prolong_add<T>, dim3(ntiles(gf)), LBLOCK, 0, st, gf, gc, mg->dir[l],
-                         (const T *)mg->x[l + 1], (T *)mg->x[l], (const T *)mg->p1[l],
+                         (const T *)mg->xres[l + 1], (T *)mg->x[l], (const T *)mg->p1[l],
                          (const T *)mg->p2[l]);
     }
     LAUNCHCHK();
     if ((rc = rbgs<T>(mg, l, 0, mg->post, st, l == 0 ? xout : nullptr, &wrote, nullptr, io)))
       return rc;
+    mg->xres[l] = mg->x[l];
   }
   if (!wrote) {
     if (io)
