@@ -46,13 +46,9 @@
 #define MG_LDS_DEFAULT (144L * 1024)   // LDS of the bottom-of-cycle workgroup
 #define CWG 1024
 #define MAX_SWEEPS 64
-#ifndef BLOCK_POINTS
-#define BLOCK_POINTS 300000L
-#endif
-#ifndef BLOCK_RATE
-#define BLOCK_RATE 50000.0
-#endif
-#define BLOCK_SWEEPS 4
+#define BLOCK_POINTS 300000L      // largest level that runs as block launches
+#define BLOCK_RATE 50000.0        // pairs the chip takes through a visit, per us
+#define BLOCK_SWEEPS 4            // most half-sweeps of a visit (the rim's width)
 
 struct LGeom {
   int n[3];
@@ -1917,7 +1913,9 @@ __global__ __launch_bounds__(CWG) void k_coarse_setup(const LevelDev<T> *__restr
 // and the sweeps.  The rim's points are recomputed by the blocks that share
 // them (each half-sweep makes one layer of it stale).  A thread keeps the
 // rows of one or two x pairs in registers; x alone goes through LDS.  Point by
-// point the operations and their order are the separate kernels'.
+// point the operations and their order are the separate kernels'.  Latency
+// bounds it: a launch, the loads, and some 0.3 us a phase; 5 to 8 us a visit
+// of up to 100,000 points, against 15 to 25 us for the launches it replaces.
 template <typename T> struct LBlock {
   LGeom g, gc;
   Mat<T> A;
@@ -2089,7 +2087,7 @@ __device__ __forceinline__ void lvl_block(const LBlock<T> &B, int blk, T *X)
     const int p = (fi - e0 + 1) + (fj - e1 + 1) * L1 + (fk - e2 + 1) * L2;
     const bool hl = f > 0, hh = f + 1 < nd;
     const T c2 = B.p2[hl ? ip - gd : ip], c1 = B.p1[hh ? ip + gd : ip];
-    const T pl = c2 * R[hl ? p - ld : p], ph = c1 * R[hh ? p + ld : p];
+    const T pl = c2 * R[hl ? p - ld : p], rh = R[hh ? p + ld : p], ph = c1 * rh;
     const T lo = hl ? pl : T(0), hi = hh ? ph : T(0);
     B.bc[(i + 1) + (j + 1) * B.gc.s[1] + (k + 1) * B.gc.s[2]] = R[p] + (lo + hi);
   }
@@ -2509,7 +2507,15 @@ static bool block_shape(const int *n, int d, const int *hl, const int *hh, size_
   return found;
 }
 
-// Which levels run as block launches.  (rule: see k_lvl_block's measurements)
+// Which levels run as block launches: symmetric storage, one to four
+// half-sweeps a visit, and at most BLOCK_POINTS points.  Below that a visit is
+// launch latency (V-cycle of 32^3 in FP64 216 us without, 103 with; 131x97x25
+// with three half-sweeps 356 and 235; 64x64x40 in FP32 with four 397 and 224);
+// above it the rims' recomputation costs more than the marching kernels' extra
+// launches.  With bounds of 150,000, 300,000 and 600,000 points the V-cycles
+// of 256x256x64 take 584, 578, 602 us (FP64, two half-sweeps) and 413, 401, 409
+// (FP32), of 131x97x25 251, 235, 286, of 512x512x64 (FP32, four half-sweeps)
+// 1475, 1447, 1440.
 static void plan_blocks(pfhip_mg *mg)
 {
   const char *e = getenv("PFHIP_MG_BLOCK");

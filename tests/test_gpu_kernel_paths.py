@@ -139,3 +139,32 @@ def test_multigrid_bottom_levels(gpu, shape, precision, sweeps):
     want = prob.interior(om.apply(b))
     tol = 1e-11 if precision == 64 else 2e-5
     assert np.max(np.abs(got - want)) <= tol * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("shape", [(32, 32, 32), (45, 33, 20), (7, 5, 60), (96, 80, 6), (130, 3, 40)])
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("sweeps", [(1, 1, 0), (2, 2, 0), (1, 1, 1), (1, 2, 0)])
+def test_multigrid_block_launches_bitwise(gpu, shape, precision, sweeps, monkeypatch):
+    """Levels visited by one block launch each against the separate launches:
+    the same bits, in the V-cycles that launch directly and that replay a
+    graph; odd extents, single-column tiles and blocks cut by the boundary.
+    The separate side restricts along z point by point: the marching form of
+    that kernel rounds one product together with the sum it enters."""
+    api = _api()
+    monkeypatch.setenv("PFHIP_MG_RRZ", "0")
+    prob = cases.hetero(*shape, seed=31)
+    gp = api.GPUProblem(prob)
+    A = cases.full_operator(prob, 32, symmetric=True)
+    bs = []
+    for q in range(3):
+        b = np.zeros(prob.shape)
+        prob.interior(b)[...] = np.random.default_rng(33 + q).normal(size=prob.interior(b).shape)
+        bs.append(b)
+    out = {}
+    for blocks in ("0", "300000"):
+        monkeypatch.setenv("PFHIP_MG_BLOCK", blocks)
+        mg = api.GPUMultigrid(gp, *sweeps, precision=precision)
+        mg.setup(A)
+        out[blocks] = [mg.apply(b) for b in bs]
+    for a, b in zip(out["0"], out["300000"]):
+        assert np.array_equal(prob.interior(a), prob.interior(b))
