@@ -3129,14 +3129,21 @@ extern "C" int pfhip_mg_apply_dq(pfhip_mg *mg, const double *b, double bscale, d
 // workgroup per member, one launch for every member with a request.  The
 // larger levels of the larger members run as grid-level phases: one launch
 // per phase and level covers that level's points of every member that has
-// it (a half-sweep, the level residual, the restriction, the prolongation,
+// it (a half-sweep, the level residual with its restriction, the prolongation,
 // the coarse operators), so no single member's one-workgroup V-cycle sets
-// the cost of every heavy round.  A launch's blocks are dealt to members in
-// segments (EnsLSeg: the member and its first block), found by a binary
-// search over the segment starts.  The per-point arithmetic is the single-
-// problem multigrid's (rbgs_point, resid_point, restrict_point,
+// the cost of every heavy round.  A table gives each workgroup of a launch its
+// member and its block of that member's points.  The per-point arithmetic is
+// the single-problem multigrid's (rbgs_point, resid_point, restrict_point,
 // prolong_point, coarse_point), in the same sweep order.
-struct EnsLSeg { int m, blk0; };
+//
+// Latency bounds a phase: 64 hillslopes hold 1.2M points, 4 us' worth of
+// traffic at most, and a phase's loads follow each other: the table, the
+// member, the level, the point.  A search of the members' first blocks in
+// place of the table took six loads more.  The table, the FP64 vectors
+// converted by the first and the last half-sweep of level 0, and the
+// restriction's loads all in flight at once took a half-sweep from 4.9 to 3.9 us
+// and two time steps of the 64 from 89.5 to 83.0 ms.
+struct EnsLSeg { int m, blk; };      // a workgroup's member and block
 
 template <typename T> struct EnsLv {
   const LevelDev<T> *lev;
@@ -3149,14 +3156,16 @@ template <typename T> struct EnsLv {
 // point sets a grid-level launch enumerates
 enum { PS_FINE = 0, PS_HALF = 1, PS_COARSE = 2, PS_N = 3 };
 enum { EL_CONV_IN, EL_FILL, EL_HALF, EL_RESTRICT, EL_PROLONG, EL_CONV_OUT, EL_COARSE };
+// with EL_HALF at level 0: convert the right-hand side first, the result last
+enum { EC_NONE = 0, EC_IN = 1, EC_OUT = 2 };
 #define ENS_LBLK 256
 
 struct pfhip_ens_mgplan {
   int n, prec, G;                     // members, level precision, grid levels
   int *lc;                            // per member: first one-workgroup level
   int pre, post, symmetric;           // the members' common sweep schedule
-  int nseg[MAXL][PS_N], nblk[MAXL][PS_N];
-  EnsLSeg *dseg[MAXL][PS_N];          // device segment tables
+  int nblk[MAXL][PS_N];
+  EnsLSeg *dseg[MAXL][PS_N];          // device tables: a phase's workgroups
   void *dM;                           // device member table EnsLv<T>[n], refilled per round
   int *dlist;                         // 0 .. n-1 (the one-workgroup kernels' members)
   int use_graph;                      // replay captured launch sequences
@@ -3173,21 +3182,42 @@ static long ens_small()
   return (e && *e) ? atol(e) : MG_SMALL_DEFAULT;
 }
 
+// resid_value at the point ip, off points from f along d, with every load
+// unconditional (the ghost layer is there to be read): the 45 loads of a
+// restriction are then in flight together, where a branch around each pair
+// made a chain of them (11 us at level 0 of 64 hillslopes, 3.3 now)
 template <typename T>
-__global__ __launch_bounds__(ENS_LBLK) void k_ens_lvl(const EnsLSeg *__restrict__ seg, int nseg,
-                                                      const EnsLv<T> *__restrict__ M, int l,
-                                                      int OP, int par, int init)
+__device__ __forceinline__ T resid_flat(const LevelDev<T> &F, int ip, const int *f, int d, int off)
 {
-  int lo = 0, hi = nseg - 1;
-  const int b = blockIdx.x;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (seg[mid].blk0 <= b) lo = mid; else hi = mid - 1;
-  }
-  const EnsLv<T> &mm = M[seg[lo].m];
+  const int i = f[0] + (d == 0 ? off : 0), j = f[1] + (d == 1 ? off : 0);
+  const int k = f[2] + (d == 2 ? off : 0);
+  const int sy = F.g.s[1], sz = F.g.s[2];
+  const T *__restrict__ x = F.x;
+  const T c = F.A.c[ip], xc = x[ip], b = F.b[ip];
+  const T aw = F.A.u[0][ip - 1], ae = F.A.u[0][ip], as = F.A.u[1][ip - sy], an = F.A.u[1][ip];
+  const T al = F.A.u[2][ip - sz], au = F.A.u[2][ip];
+  const T xw = x[ip - 1], xe = x[ip + 1], xs = x[ip - sy], xn = x[ip + sy];
+  const T xl = x[ip - sz], xu = x[ip + sz];
+  T v = c * xc;
+  v = b_fma(i > 0 ? aw : T(0), xw, v);
+  v = b_fma(i + 1 < F.g.n[0] ? ae : T(0), xe, v);
+  v = b_fma(j > 0 ? as : T(0), xs, v);
+  v = b_fma(j + 1 < F.g.n[1] ? an : T(0), xn, v);
+  v = b_fma(k > 0 ? al : T(0), xl, v);
+  v = b_fma(k + 1 < F.g.n[2] ? au : T(0), xu, v);
+  return b - v;
+}
+
+template <typename T>
+__global__ __launch_bounds__(ENS_LBLK) void k_ens_lvl(const EnsLSeg *__restrict__ seg,
+                                                      const EnsLv<T> *__restrict__ M, int l,
+                                                      int OP, int par, int init, int conv)
+{
+  const EnsLSeg sg = seg[blockIdx.x];
+  const EnsLv<T> &mm = M[sg.m];
   if (!mm.act) return;
   const LevelDev<T> &F = mm.lev[l];
-  const int idx = (b - seg[lo].blk0) * ENS_LBLK + threadIdx.x;
+  const int idx = sg.blk * ENS_LBLK + threadIdx.x;
   int i, j, k;
   if (OP == EL_HALF) {
     const int nx = F.g.n[0], ny = F.g.n[1], nz = F.g.n[2];
@@ -3195,9 +3225,19 @@ __global__ __launch_bounds__(ENS_LBLK) void k_ens_lvl(const EnsLSeg *__restrict_
     if (idx >= ncol * ny * nz) return;
     const int t = idx % ncol, r = idx / ncol;
     j = r % ny; k = r / ny;
-    i = ((par - j - k) & 1) + 2 * t;
-    if (i >= nx) return;
-    rbgs_point<T, false>(F.g, F.A, F.x, F.b, par, init, i, j, k);
+    const int odd = (par - j - k) & 1;
+    i = odd + 2 * t;
+    // the pair's point of the other colour
+    const int io = (odd ^ 1) + 2 * t;
+    if (conv == EC_IN) {
+      if (i < nx) { const long ip = LIDX(F.g, i, j, k); F.b[ip] = (T)mm.bin[ip]; }
+      if (io < nx) { const long ip = LIDX(F.g, io, j, k); F.b[ip] = (T)mm.bin[ip]; }
+    }
+    if (i < nx) rbgs_point<T, false>(F.g, F.A, F.x, F.b, par, init, i, j, k);
+    if (conv == EC_OUT) {
+      if (i < nx) { const long ip = LIDX(F.g, i, j, k); mm.xout[ip] = (double)F.x[ip]; }
+      if (io < nx) { const long ip = LIDX(F.g, io, j, k); mm.xout[ip] = (double)F.x[ip]; }
+    }
     return;
   }
   if (OP == EL_RESTRICT || OP == EL_COARSE) {
@@ -3206,24 +3246,20 @@ __global__ __launch_bounds__(ENS_LBLK) void k_ens_lvl(const EnsLSeg *__restrict_
     unflat(Cc.g, idx, i, j, k);
     if (OP == EL_RESTRICT) {
       // the fine residuals at C-1, C, C+1 in place (k_resid_restrict's
-      // expressions), so no separate residual phase
+      // expressions), so no separate residual phase; a missing neighbour's
+      // loads go to C
       int f[3] = { i, j, k };
       const int d = F.dir;
       f[d] *= 2;
-      const long iF = LIDX(F.g, f[0], f[1], f[2]);
-      const long sd = F.g.s[d];
-      const T rC = resid_value<T, false>(F.g, F.A, F.x, F.b, f[0], f[1], f[2]);
-      T rlo = T(0), rhi = T(0);
-      if (f[d] > 0) {
-        int q[3] = { f[0], f[1], f[2] };
-        q[d] -= 1;
-        rlo = F.p2[iF - sd] * resid_value<T, false>(F.g, F.A, F.x, F.b, q[0], q[1], q[2]);
-      }
-      if (f[d] + 1 < F.g.n[d]) {
-        int q[3] = { f[0], f[1], f[2] };
-        q[d] += 1;
-        rhi = F.p1[iF + sd] * resid_value<T, false>(F.g, F.A, F.x, F.b, q[0], q[1], q[2]);
-      }
+      const bool hl = f[d] > 0, hh = f[d] + 1 < F.g.n[d];
+      const int sd = d == 0 ? 1 : F.g.s[d], iF = (int)LIDX(F.g, f[0], f[1], f[2]);
+      const int iL = hl ? iF - sd : iF, iH = hh ? iF + sd : iF;
+      const T c2 = F.p2[iL], c1 = F.p1[iH];
+      const T rC = resid_flat<T>(F, iF, f, d, 0);
+      const T rL = resid_flat<T>(F, iL, f, d, hl ? -1 : 0);
+      const T rH = resid_flat<T>(F, iH, f, d, hh ? 1 : 0);
+      const T vlo = c2 * rL, vhi = c1 * rH;
+      const T rlo = hl ? vlo : T(0), rhi = hh ? vhi : T(0);
       Cc.b[LIDX(Cc.g, i, j, k)] = rC + (rlo + rhi);
     }
     else
@@ -3312,14 +3348,23 @@ extern "C" int pfhip_ens_mg_plan_destroy(pfhip_ens_mgplan *p)
   return PFHIP_OK;
 }
 
+static int ens_table(void **d, const void *h, size_t bytes)
+{
+  int rc = pfhip_malloc(d, (long)bytes);
+  if (rc == PFHIP_OK && hipMemcpy(*d, h, bytes, hipMemcpyHostToDevice) != hipSuccess) {
+    pfhip_set_error("hipMemcpy of an ensemble table");
+    rc = PFHIP_ERR_HIP;
+  }
+  return rc;
+}
+
 extern "C" int pfhip_ens_mg_plan_create(pfhip_mg *const *mgs, int n, pfhip_ens_mgplan **out)
 {
   pfhip_ens_mgplan *p = (pfhip_ens_mgplan *)calloc(1, sizeof(pfhip_ens_mgplan));
   int *order = (int *)malloc(sizeof(int) * (size_t)n);
-  EnsLSeg *h = (EnsLSeg *)malloc(sizeof(EnsLSeg) * (size_t)n);
   if (p) p->lc = (int *)malloc(sizeof(int) * (size_t)n);
-  if (!p || !order || !h || !p->lc) {
-    free(order); free(h); pfhip_ens_mg_plan_destroy(p);
+  if (!p || !order || !p->lc) {
+    free(order); pfhip_ens_mg_plan_destroy(p);
     pfhip_set_error("out of host memory");
     return PFHIP_ERR_NOMEM;
   }
@@ -3391,24 +3436,22 @@ extern "C" int pfhip_ens_mg_plan_create(pfhip_mg *const *mgs, int n, pfhip_ens_m
   }
   for (int l = 0; l < p->G && rc == PFHIP_OK; l++) {
     for (int s = 0; s < PS_N && rc == PFHIP_OK; s++) {
-      int ns = 0, nb = 0;
+      long nb = 0;
+      for (int m = 0; m < n; m++)
+        if (p->lc[m] > l) nb += (ps_points(mgs[m], l, s) + ENS_LBLK - 1) / ENS_LBLK;
+      p->nblk[l][s] = (int)nb;
+      if (nb == 0) continue;
+      EnsLSeg *h = (EnsLSeg *)malloc(sizeof(EnsLSeg) * (size_t)nb);
+      if (!h) { pfhip_set_error("out of host memory"); rc = PFHIP_ERR_NOMEM; break; }
+      long at = 0;
       for (int q = 0; q < n; q++) {
         const int m = order[q];
         if (p->lc[m] <= l) continue;
-        h[ns].m = m;
-        h[ns].blk0 = nb;
-        nb += (int)((ps_points(mgs[m], l, s) + ENS_LBLK - 1) / ENS_LBLK);
-        ns++;
+        const long mb = (ps_points(mgs[m], l, s) + ENS_LBLK - 1) / ENS_LBLK;
+        for (long b = 0; b < mb; b++, at++) { h[at].m = m; h[at].blk = (int)b; }
       }
-      p->nseg[l][s] = ns;
-      p->nblk[l][s] = nb;
-      if (ns == 0) continue;
-      rc = pfhip_malloc((void **)&p->dseg[l][s], (long)sizeof(EnsLSeg) * ns);
-      if (rc == PFHIP_OK &&
-          hipMemcpy(p->dseg[l][s], h, sizeof(EnsLSeg) * ns, hipMemcpyHostToDevice) != hipSuccess) {
-        pfhip_set_error("hipMemcpy of an ensemble segment table");
-        rc = PFHIP_ERR_HIP;
-      }
+      rc = ens_table((void **)&p->dseg[l][s], h, sizeof(EnsLSeg) * (size_t)nb);
+      free(h);
     }
   }
   const size_t mb = (size_t)n * (p->prec == 32 ? sizeof(EnsLv<float>) : sizeof(EnsLv<double>));
@@ -3427,30 +3470,38 @@ extern "C" int pfhip_ens_mg_plan_create(pfhip_mg *const *mgs, int n, pfhip_ens_m
     rc = PFHIP_ERR_HIP;
   }
   free(order);
-  free(h);
   if (rc) { pfhip_ens_mg_plan_destroy(p); return rc; }
   *out = p;
   return PFHIP_OK;
 }
 
 template <typename T>
-static void ens_phase(pfhip_ens_mgplan *p, int l, int ps, int op, int par, int init,
+static void ens_phase(pfhip_ens_mgplan *p, int l, int ps, int op, int par, int init, int conv,
                       hipStream_t s)
 {
   if (p->nblk[l][ps] == 0) return;
   p->launches++;
   hipLaunchKernelGGL(k_ens_lvl<T>, dim3(p->nblk[l][ps]), dim3(ENS_LBLK), 0, s, p->dseg[l][ps],
-                     p->nseg[l][ps], (const EnsLv<T> *)p->dM, l, op, par, init);
+                     (const EnsLv<T> *)p->dM, l, op, par, init, conv);
 }
 
+// conv: the conversion that the first (EC_IN) or the last (EC_OUT) half-sweep
+// takes along
 template <typename T>
-static void ens_sweeps(pfhip_ens_mgplan *p, int l, int zero, int max_iter, hipStream_t s)
+static void ens_sweeps(pfhip_ens_mgplan *p, int l, int zero, int max_iter, int conv,
+                       hipStream_t s)
 {
   HalfSweep seq[2 * MAX_SWEEPS + 4];
   int fill;
   const int ns = sweep_list(p->symmetric, zero, max_iter, seq, &fill);
-  if (fill) ens_phase<T>(p, l, PS_FINE, EL_FILL, 0, 0, s);
-  for (int q = 0; q < ns; q++) ens_phase<T>(p, l, PS_HALF, EL_HALF, seq[q].par, seq[q].init, s);
+  const bool alone = conv == EC_IN ? ns == 0 || fill : ns == 0;
+  if (alone && conv == EC_IN) ens_phase<T>(p, l, PS_FINE, EL_CONV_IN, 0, 0, 0, s);
+  if (fill) ens_phase<T>(p, l, PS_FINE, EL_FILL, 0, 0, 0, s);
+  for (int q = 0; q < ns; q++) {
+    const bool here = !alone && q == (conv == EC_IN ? 0 : ns - 1);
+    ens_phase<T>(p, l, PS_HALF, EL_HALF, seq[q].par, seq[q].init, here ? conv : EC_NONE, s);
+  }
+  if (alone && conv == EC_OUT) ens_phase<T>(p, l, PS_FINE, EL_CONV_OUT, 0, 0, 0, s);
 }
 
 // The launch sequence of one round: the coarse operators (apply = 0) or one
@@ -3463,7 +3514,7 @@ static int ens_sequence(pfhip_ens_mgplan *p, int apply, hipStream_t s)
   const EnsLv<T> *dM = (const EnsLv<T> *)p->dM;
   if (!apply) {
     for (int l = 0; l < p->G; l++) {
-      ens_phase<T>(p, l, PS_COARSE, EL_COARSE, 0, 0, s);
+      ens_phase<T>(p, l, PS_COARSE, EL_COARSE, 0, 0, 0, s);
       LAUNCHCHK();
     }
     hipLaunchKernelGGL(k_ens_mg_coarse<T>, dim3(p->n), dim3(CWG), 0, s, dM, p->dlist);
@@ -3471,10 +3522,9 @@ static int ens_sequence(pfhip_ens_mgplan *p, int apply, hipStream_t s)
     p->launches++;
     return PFHIP_OK;
   }
-  if (p->G > 0) ens_phase<T>(p, 0, PS_FINE, EL_CONV_IN, 0, 0, s);
   for (int l = 0; l < p->G; l++) {
-    ens_sweeps<T>(p, l, 1, p->pre, s);
-    ens_phase<T>(p, l, PS_COARSE, EL_RESTRICT, 0, 0, s);
+    ens_sweeps<T>(p, l, 1, p->pre, l == 0 ? EC_IN : EC_NONE, s);
+    ens_phase<T>(p, l, PS_COARSE, EL_RESTRICT, 0, 0, 0, s);
     LAUNCHCHK();
   }
   if (p->lds_bytes > 0)
@@ -3485,12 +3535,10 @@ static int ens_sequence(pfhip_ens_mgplan *p, int apply, hipStream_t s)
   LAUNCHCHK();
   p->launches++;
   for (int l = p->G - 1; l >= 0; l--) {
-    ens_phase<T>(p, l, PS_FINE, EL_PROLONG, 0, 0, s);
-    ens_sweeps<T>(p, l, 0, p->post, s);
+    ens_phase<T>(p, l, PS_FINE, EL_PROLONG, 0, 0, 0, s);
+    ens_sweeps<T>(p, l, 0, p->post, l == 0 ? EC_OUT : EC_NONE, s);
     LAUNCHCHK();
   }
-  if (p->G > 0) ens_phase<T>(p, 0, PS_FINE, EL_CONV_OUT, 0, 0, s);
-  LAUNCHCHK();
   return PFHIP_OK;
 }
 
