@@ -8,9 +8,9 @@
  * call as a request and switches back to the scheduler.  Once every live
  * member has a request pending, the scheduler serves them by kind with one
  * batched launch each (all vector operations and reductions together, all
- * residual forms, all PC setups, all V-cycles), copies the reduction
- * results back with one transfer and one synchronisation, and resumes the
- * members it served.  PC setups and V-cycles are held back while lighter
+ * residual forms, all PC setups, all V-cycles), waits for the reduction
+ * results, which the device writes to pinned memory, and resumes the members
+ * it served.  PC setups and V-cycles are held back while lighter
  * requests are pending, which keeps the members in step.  A member whose steps are done leaves the rotation: the set of
  * live members is the convergence mask of every launch.
  *
@@ -86,7 +86,7 @@ struct pfhip_ensemble {
   ens_member *m;
   void *sched_sp;
   int cur;
-  double *d_res, *h_res;
+  pfhip_ens_results res;
   double *d_part;                       /* block partials of vector ops    */
   pfhip_ens_stage st;
   pfhip_ens_req **lists[PFHIP_EOP_COUNT];
@@ -307,7 +307,7 @@ static int e_saturation(pfhip_problem *pb, const double *p, double *out, int fcn
   return submit();
 }
 
-/* results reach a member only through the scheduler's synchronised copy;
+/* results reach a member only through the scheduler, which waits for them;
  * a synchronisation point only has to launch what is queued */
 static int e_synchronize(void) { return flush(); }
 
@@ -329,9 +329,8 @@ int pfhip_ensemble_destroy(pfhip_ensemble *e)
     free(m->stack);
     if (m->s) pfhip_solver_set_ops(m->s, &pfhip_direct_ops);
   }
-  pfhip_free(e->d_res);
   pfhip_free(e->d_part);
-  pfhip_host_free(e->h_res);
+  pfhip_ens_results_destroy(&e->res);
   pfhip_ens_stage_destroy(&e->st);
   pfhip_ens_mg_plan_destroy(e->mgplan);
   for (int k = 0; k < PFHIP_EOP_COUNT; k++) free(e->lists[k]);
@@ -391,8 +390,7 @@ int pfhip_ensemble_create(int n, pfhip_solver *const *solvers, pfhip_ensemble **
   long blocks = 0;
   for (int i = 0; i < n && !rc; i++) blocks += pfhip_ens_vec_blocks(e->m[i].pb->ncell);
   if (!rc) rc = pfhip_dev_alloc(&e->d_part, blocks * PFHIP_ENS_NRES);
-  if (!rc) rc = pfhip_dev_alloc(&e->d_res, (long)n * ENS_QMAX * PFHIP_ENS_NRES);
-  if (!rc) rc = pfhip_host_alloc(&e->h_res, (long)n * ENS_QMAX * PFHIP_ENS_NRES);
+  if (!rc) rc = pfhip_ens_results_create(&e->res, (long)n * ENS_QMAX * PFHIP_ENS_NRES);
   if (!rc) rc = pfhip_ens_stage_create(&e->st, ENS_STAGE);
   if (!rc) {
     pfhip_mg **mgs = (pfhip_mg **)malloc(sizeof(pfhip_mg *) * (size_t)n);
@@ -455,7 +453,7 @@ static void set_rc(pfhip_ens_req **l, int n, int rc)
 
 /* Serve the queued requests of this round, position by position (a
  * member's queue runs in its order; every position is one launch per kind
- * across the members), then fetch all results with one copy.  The heavy
+ * across the members), then wait once for all results.  The heavy
  * kinds (PC setup, V-cycle: their cost is set by the largest member, not by
  * how many members take part) wait while any light request is queued: the
  * members that are behind catch up through light rounds, and each heavy
@@ -475,7 +473,7 @@ static int serve_round(pfhip_ensemble *e)
     if (light && is_heavy(m->q[m->qlen - 1].op)) m->nexec--;   /* deferred */
     if (m->nexec > maxp) maxp = m->nexec;
   }
-  int slots = 0, nouts = 0;
+  int slots = 0, nouts = 0, behind = 0;
   for (int pos = 0; pos < maxp; pos++) {
     int nv = 0;
     for (int k = 0; k < PFHIP_EOP_COUNT; k++) e->nlist[k] = 0;
@@ -492,12 +490,14 @@ static int serve_round(pfhip_ensemble *e)
       }
     }
     if (nv) {
-      rc = pfhip_ens_exec_vec(e->vec, nv, e->d_res + (long)slots * PFHIP_ENS_NRES, e->d_part,
-                              &e->st, NULL);
+      int gives = 0;
+      rc = pfhip_ens_exec_vec(e->vec, nv, &e->res, slots, e->d_part, &e->st, NULL, &gives);
+      behind = !gives;
       set_rc(e->vec, nv, rc);
       slots += nv;
       e->launches++;
     }
+    for (int k = 0; k < PFHIP_EOP_COUNT; k++) if (e->nlist[k]) behind = 1;
     int nr = e->nlist[PFHIP_EOP_RESIDUAL];
     if (nr) {
       rc = pfhip_ens_exec_residual(e->lists[PFHIP_EOP_RESIDUAL], nr, &e->st, NULL);
@@ -535,13 +535,15 @@ static int serve_round(pfhip_ensemble *e)
   }
   int frc = PFHIP_OK;
   if (nouts) {
-    frc = pfhip_ens_fetch(e->h_res, e->d_res, (long)slots * PFHIP_ENS_NRES, NULL);
+    frc = pfhip_ens_results_wait(&e->res, NULL);
     if (frc == PFHIP_OK) {
-      e->st.off = 0;
+      /* the ring starts over unless launches queued after the last results
+       * still read their tables */
+      if (!behind) e->st.off = 0;
       for (int v = 0; v < nouts; v++) {
         pfhip_ens_req *r = e->outs[v];
         for (int k = 0; k < r->nout; k++)
-          *r->out[k] = e->h_res[(long)r->slot * PFHIP_ENS_NRES + k];
+          *r->out[k] = e->res.host[(long)r->slot * PFHIP_ENS_NRES + k];
       }
     }
   }

@@ -3454,7 +3454,9 @@ extern "C" int pfhip_ens_mg_plan_create(pfhip_mg *const *mgs, int n, pfhip_ens_m
       free(h);
     }
   }
-  const size_t mb = (size_t)n * (p->prec == 32 ? sizeof(EnsLv<float>) : sizeof(EnsLv<double>));
+  // whole 16-byte units, as pfhip_ens_commit_to copies them
+  const size_t mb = ((size_t)n * (p->prec == 32 ? sizeof(EnsLv<float>) : sizeof(EnsLv<double>)) +
+                     15) & ~(size_t)15;
   if (rc == PFHIP_OK) rc = pfhip_malloc(&p->dM, (long)mb);
   if (rc == PFHIP_OK) rc = pfhip_malloc((void **)&p->dlist, (long)sizeof(int) * n);
   if (rc == PFHIP_OK) {
@@ -3574,7 +3576,7 @@ static int ens_mg_launch(pfhip_ens_mgplan *p, pfhip_ens_req *const *rq, int n, i
                          pfhip_ens_stage *st, hipStream_t s)
 {
   // the member table of this round: every member inactive but those with a
-  // request; staged through the ring, then copied to the plan's fixed table
+  // request; staged through the ring, copied to the plan's fixed table
   const long mbytes = (long)sizeof(EnsLv<T>) * p->n;
   EnsLv<T> *M = (EnsLv<T> *)pfhip_ens_reserve(st, mbytes, s);
   if (!M) return PFHIP_ERR_HIP;
@@ -3595,9 +3597,8 @@ static int ens_mg_launch(pfhip_ens_mgplan *p, pfhip_ens_req *const *rq, int n, i
     e.pre = mg->pre; e.post = mg->post; e.symmetric = mg->symmetric;
     e.act = 1;
   }
-  void *dstage = pfhip_ens_commit(st, mbytes, s);
-  if (!dstage) return PFHIP_ERR_HIP;
-  HIPCHK(hipMemcpyAsync(p->dM, dstage, (size_t)mbytes, hipMemcpyDeviceToDevice, s));
+  const int urc = pfhip_ens_commit_to(st, p->dM, mbytes, s);
+  if (urc) return urc;
   if (p->use_graph) {
     if (!p->gx[apply]) {
       int rc = ens_capture<T>(p, apply);

@@ -261,14 +261,27 @@ typedef struct pfhip_ens_stage {
   long off, cap;
 } pfhip_ens_stage;
 
-void *pfhip_ens_upload(pfhip_ens_stage *st, const void *src, long bytes, void *stream);
-/* in-place form: reserve returns the host address to fill, commit copies it
- * and returns the device address */
+/* results of a round's requests: pinned slots the device writes, and the
+ * number of the last launch whose results are there */
+typedef struct pfhip_ens_results {
+  double *host;
+  unsigned long long *flag, seq;
+  unsigned *ticket;
+} pfhip_ens_results;
+int pfhip_ens_results_create(pfhip_ens_results *r, long n);
+void pfhip_ens_results_destroy(pfhip_ens_results *r);
+int pfhip_ens_results_wait(pfhip_ens_results *r, void *stream);
+
+/* tables are filled in place: reserve returns the host address, commit copies
+ * to the ring's device twin and returns that address, or to dst */
 void *pfhip_ens_reserve(pfhip_ens_stage *st, long bytes, void *stream);
 void *pfhip_ens_commit(pfhip_ens_stage *st, long bytes, void *stream);
-/* batched launches; results of request r land in res[r * PFHIP_ENS_NRES + v] */
-int pfhip_ens_exec_vec(pfhip_ens_req *const *rq, int n, double *res, double *part,
-                       pfhip_ens_stage *st, void *stream);
+int pfhip_ens_commit_to(pfhip_ens_stage *st, void *dst, long bytes, void *stream);
+/* batched launches; results of request r land in
+ * res->host[(slot + r) * PFHIP_ENS_NRES + v] once pfhip_ens_results_wait
+ * returns; *results: whether the launch hands any over */
+int pfhip_ens_exec_vec(pfhip_ens_req *const *rq, int n, pfhip_ens_results *res, long slot,
+                       double *part, pfhip_ens_stage *st, void *stream, int *results);
 /* blocks of the flat vector grid for a member of ncell cells; part needs
  * PFHIP_ENS_NRES doubles per block */
 long pfhip_ens_vec_blocks(long ncell);
@@ -298,10 +311,6 @@ int pfhip_mg_pair_shapes(pfhip_mg *mg, int *shape, int max);
 void pfhip_mg_level0(pfhip_mg *mg, void **A, int *prec);
 int pfhip_ens_stage_create(pfhip_ens_stage *st, long cap);
 void pfhip_ens_stage_destroy(pfhip_ens_stage *st);
-/* n doubles device -> pinned host, then a stream synchronisation */
-int pfhip_ens_fetch(double *host, const double *dev, long n, void *stream);
-int pfhip_host_alloc(double **p, long n);
-void pfhip_host_free(double *p);
 
 #ifdef __cplusplus
 }
