@@ -3788,13 +3788,25 @@ struct EnsVec {
   double *z;
 };
 
-// Vector operations as a flat grid: block b takes EVC consecutive interior
-// cells of one member (EVB threads, EVC / EVB cells each, a fixed mapping)
-// and writes its partial results to part[b * PFHIP_ENS_NRES + v]; the
-// finishing kernel then adds (or maxes) each member's block partials in
-// block order, so the results are reproducible bit for bit.
+// Vector operations as a flat grid: a block takes EVC consecutive interior
+// cells of one member (EVB threads, EVU cells each, a fixed mapping) and writes
+// its partial results to part[block * PFHIP_ENS_NRES + v]; the finishing kernel
+// then adds (or maxes) each member's block partials in block order, so the
+// results are reproducible bit for bit.
+//
+// Latency bounds it: 64 hillslopes are 10 MB a vector, and what counts is how
+// many loads follow each other.  A table gives the block its request; a thread
+// places its cells with one division and steps, and holds all of them, so a
+// linear combination's or a multi-dot's term is EVU loads in flight and its
+// pointer is read once, ENS_QU terms at a time; a multi-dot adds up its
+// wavefronts in LDS behind one barrier.  Two time steps of 64 hillslopes: 76.8 ms
+// with a search for the request, a division per cell and a barrier pair per dot
+// product; 72.2, 71.7, 71.0 with 8, 4, 2 cells a thread (of 12 hillslopes 30.9;
+// 28.9, 28.4, 28.5).
 #define EVB 256
-#define EVC 2048
+#define EVU 4
+#define EVC (EVB * EVU)
+#define ENS_QU 4
 
 __device__ __forceinline__ bool ens_is_max(int op)
 {
@@ -3812,85 +3824,158 @@ __device__ __forceinline__ int ens_nres(const EnsVec &E)
   }
 }
 
-#define ENS_MDOT 32
 __global__ __launch_bounds__(EVB) void k_ens_vec(const EnsVec *__restrict__ T,
-                                                 const int *__restrict__ starts, int n,
+                                                 const int2 *__restrict__ blocks,
                                                  const double *__restrict__ QC,
                                                  const double *const *__restrict__ QX,
                                                  double *__restrict__ part)
 {
-  const int e = ens_find(starts, n, blockIdx.x);
-  const EnsVec &E = T[e];
+  const int2 bk = blocks[blockIdx.x];          // request, block of its member
+  const EnsVec &E = T[bk.x];
   const double *__restrict__ Ec = QC + E.qoff;
   const double *const *__restrict__ Ex = QX + E.qoff;
   const Geom g = E.g;
-  const int op = E.op, nq = E.nq;
-  const int c0 = (blockIdx.x - starts[e]) * EVC;
-  const int c1 = min(c0 + EVC, E.ncell);
+  const int op = E.op, nq = E.nq, base = E.base, norm = E.norm;
+  const double cst = E.cst;
+  double *z = E.z;
   double *P = part + (long)blockIdx.x * PFHIP_ENS_NRES;
+  // the thread's cells c0 + thread + u EVB; past the end, the block's first
+  const int c0 = bk.y * EVC, left = min(EVC, E.ncell - c0) - (int)threadIdx.x;
+  const int dr = EVB / g.nx, di = EVB - dr * g.nx, dk = dr / g.ny, dj = dr - dk * g.ny;
   int i, j, k;
+  const int first = cell_ip(g, c0, i, j, k);
+  int ip[EVU];
+  bool ok[EVU];
+  cell_ip(g, c0 + threadIdx.x, i, j, k);
+#pragma unroll
+  for (int u = 0; u < EVU; u++) {
+    ok[u] = u * EVB < left;
+    ip[u] = ok[u] ? (i + 1) + (j + 1) * g.sy + (k + 1) * g.sz : first;
+    i += di;
+    int c = i >= g.nx;
+    i -= c ? g.nx : 0;
+    j += dj + c;
+    c = j >= g.ny;
+    j -= c ? g.ny : 0;
+    k += dk + c;
+  }
   if (op == PFHIP_EOP_LIN) {
     // z may alias an input: every cell is read before it is written, by
     // the same thread
-    double acc = 0.0;
-    for (int c = c0 + threadIdx.x; c < c1; c += EVB) {
-      const int ip = cell_ip(g, c, i, j, k);
-      double s;
-      int q0;
-      if (E.base) { s = E.z[ip]; q0 = 0; }
-      else if (nq > 0) { s = Ec[0] * Ex[0][ip]; q0 = 1; }
-      else { s = E.cst; q0 = 0; }
-      for (int q = q0; q < nq; q++) s += Ec[q] * Ex[q][ip];
-      E.z[ip] = s;
-      acc += s * s;
+    double s[EVU], acc = 0.0;
+    int q = 0;
+#pragma unroll
+    for (int u = 0; u < EVU; u++) s[u] = cst;
+    if (base) {
+#pragma unroll
+      for (int u = 0; u < EVU; u++) s[u] = z[ip[u]];
+    } else if (nq > 0) {
+      const double c = Ec[0];
+      const double *x = Ex[0];
+#pragma unroll
+      for (int u = 0; u < EVU; u++) s[u] = c * x[ip[u]];
+      q = 1;
     }
-    if (E.norm) {
+    for (; q + ENS_QU <= nq; q += ENS_QU) {
+      double v[ENS_QU][EVU];
+#pragma unroll
+      for (int t = 0; t < ENS_QU; t++) {
+        const double *x = Ex[q + t];
+#pragma unroll
+        for (int u = 0; u < EVU; u++) v[t][u] = x[ip[u]];
+      }
+#pragma unroll
+      for (int t = 0; t < ENS_QU; t++) {
+        const double c = Ec[q + t];
+#pragma unroll
+        for (int u = 0; u < EVU; u++) s[u] += c * v[t][u];
+      }
+    }
+    for (; q < nq; q++) {
+      const double c = Ec[q];
+      const double *x = Ex[q];
+#pragma unroll
+      for (int u = 0; u < EVU; u++) s[u] += c * x[ip[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < EVU; u++)
+      if (ok[u]) {
+        z[ip[u]] = s[u];
+        acc += s[u] * s[u];
+      }
+    if (norm) {
       acc = block_reduce<false>(acc);
       if (threadIdx.x == 0) P[0] = acc;
     }
     return;
   }
   if (op == PFHIP_EOP_MDOT) {
-    double acc[ENS_MDOT];
+    __shared__ double sh[PFHIP_ENS_NRES][EVB / 64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    double w[EVU];
 #pragma unroll
-    for (int q = 0; q < ENS_MDOT; q++) acc[q] = 0.0;
-    for (int c = c0 + threadIdx.x; c < c1; c += EVB) {
-      const int ip = cell_ip(g, c, i, j, k);
-      const double w = E.y[ip];
+    for (int u = 0; u < EVU; u++) w[u] = E.y[ip[u]];
+    for (int q = 0; q < nq; q += ENS_QU) {
+      double v[ENS_QU][EVU];
 #pragma unroll
-      for (int q = 0; q < ENS_MDOT; q++)
-        if (q < nq) acc[q] += Ex[q][ip] * w;
-    }
+      for (int t = 0; t < ENS_QU; t++) {
+        const double *x = Ex[min(q + t, nq - 1)];
 #pragma unroll
-    for (int q = 0; q < ENS_MDOT; q++) {
-      if (q < nq) {
-        double s = block_reduce<false>(acc[q]);
-        if (threadIdx.x == 0) P[q] = s;
+        for (int u = 0; u < EVU; u++) v[t][u] = x[ip[u]];
       }
+#pragma unroll
+      for (int t = 0; t < ENS_QU; t++) {
+        double a = 0.0;
+#pragma unroll
+        for (int u = 0; u < EVU; u++) a = ok[u] ? fma(v[t][u], w[u], a) : a;
+        a = wave_sum(a);
+        if (lane == 0 && q + t < nq) sh[q + t][wv] = a;
+      }
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nq) {
+      double r = sh[threadIdx.x][0];
+#pragma unroll
+      for (int h = 1; h < EVB / 64; h++) r += sh[threadIdx.x][h];
+      P[threadIdx.x] = r;
     }
     return;
   }
   double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-  for (int c = c0 + threadIdx.x; c < c1; c += EVB) {
-    const int ip = cell_ip(g, c, i, j, k);
-    switch (op) {
-      case PFHIP_EOP_DOT: a0 += E.x[ip] * E.y[ip]; break;
-      case PFHIP_EOP_MAXABS: a0 = fmax(a0, fabs(E.x[ip])); break;
-      case PFHIP_EOP_SCSTEP: a0 = fmax(a0, fabs(E.y[ip] / (1.0 + fabs(E.x[ip])))); break;
-      case PFHIP_EOP_DQ: {
-        double u = E.x[ip], v = E.y[ip];
-        a0 += u * v;
-        a1 += v * v;
-        a2 += fabs(v);
-        break;
+  double x[EVU], y[EVU];
+  const bool two = op != PFHIP_EOP_MAXABS;
+#pragma unroll
+  for (int u = 0; u < EVU; u++) x[u] = E.x[ip[u]];
+#pragma unroll
+  for (int u = 0; u < EVU; u++) y[u] = two ? E.y[ip[u]] : 0.0;
+  switch (op) {
+    case PFHIP_EOP_DOT:
+#pragma unroll
+      for (int u = 0; u < EVU; u++) a0 = ok[u] ? fma(x[u], y[u], a0) : a0;
+      break;
+    case PFHIP_EOP_MAXABS:
+#pragma unroll
+      for (int u = 0; u < EVU; u++) a0 = ok[u] ? fmax(a0, fabs(x[u])) : a0;
+      break;
+    case PFHIP_EOP_SCSTEP:
+#pragma unroll
+      for (int u = 0; u < EVU; u++) a0 = ok[u] ? fmax(a0, fabs(y[u] / (1.0 + fabs(x[u])))) : a0;
+      break;
+    case PFHIP_EOP_DQ:
+#pragma unroll
+      for (int u = 0; u < EVU; u++) {
+        a0 = ok[u] ? fma(x[u], y[u], a0) : a0;
+        a1 = ok[u] ? fma(y[u], y[u], a1) : a1;
+        a2 = ok[u] ? a2 + fabs(y[u]) : a2;
       }
-      default: {   // PFHIP_EOP_STOP
-        a0 = fmax(a0, fabs(E.x[ip]));
-        double un = E.y[ip];
-        double st = 1.0 * un + (-1.0) * E.u[ip];
-        a1 = fmax(a1, fabs(st / (1.0 + fabs(un))));
+      break;
+    default:   // PFHIP_EOP_STOP
+#pragma unroll
+      for (int u = 0; u < EVU; u++) {
+        const double st = 1.0 * y[u] + (-1.0) * E.u[ip[u]];
+        a0 = ok[u] ? fmax(a0, fabs(x[u])) : a0;
+        a1 = ok[u] ? fmax(a1, fabs(st / (1.0 + fabs(y[u])))) : a1;
       }
-    }
   }
   const bool mx = ens_is_max(op);
   a0 = mx ? block_reduce<true>(a0) : block_reduce<false>(a0);
@@ -4027,16 +4112,19 @@ extern "C" int pfhip_ens_exec_vec(pfhip_ens_req *const *rq, int n, pfhip_ens_res
   if (n <= 0) return PFHIP_OK;
   long nqt = 0;
   for (int r = 0; r < n; r++) nqt += rq[r]->nq;
-  // one table upload: entries | block starts | term coefficients | term pointers
+  long blocks = 0;
+  for (int r = 0; r < n; r++) blocks += pfhip_ens_vec_blocks(rq[r]->pb->ncell);
+  // one table upload: entries | block starts | blocks | term coefficients | term pointers
   const long bT = al256((long)n * sizeof(EnsVec)), bS = al256((long)(n + 1) * sizeof(int));
-  const long bC = al256(nqt * (long)sizeof(double));
-  const long bytes = bT + bS + bC + al256(nqt * (long)sizeof(void *));
+  const long bB = al256(blocks * (long)sizeof(int2)), bC = al256(nqt * (long)sizeof(double));
+  const long bytes = bT + bS + bB + bC + al256(nqt * (long)sizeof(void *));
   char *h = (char *)pfhip_ens_reserve(st, bytes, stream);
   if (!h) return PFHIP_ERR_HIP;
   EnsVec *T = (EnsVec *)h;
   int *starts = (int *)(h + bT);
-  double *QC = (double *)(h + bT + bS);
-  const double **QX = (const double **)(h + bT + bS + bC);
+  int2 *bk = (int2 *)(h + bT + bS);
+  double *QC = (double *)(h + bT + bS + bB);
+  const double **QX = (const double **)(h + bT + bS + bB + bC);
   int blk = 0, give = 0;
   long qo = 0;
   for (int r = 0; r < n; r++) {
@@ -4050,7 +4138,9 @@ extern "C" int pfhip_ens_exec_vec(pfhip_ens_req *const *rq, int n, pfhip_ens_res
     for (int t = 0; t < q->nq; t++) { QC[qo + t] = q->c[t]; QX[qo + t] = q->xq[t]; }
     qo += q->nq;
     starts[r] = blk;
-    blk += (int)((q->pb->ncell + EVC - 1) / EVC);
+    const int nb = (int)pfhip_ens_vec_blocks(q->pb->ncell);
+    for (int b = 0; b < nb; b++) bk[blk + b] = make_int2(r, b);
+    blk += nb;
     if (q->nout) give = 1;
   }
   starts[n] = blk;
@@ -4058,9 +4148,9 @@ extern "C" int pfhip_ens_exec_vec(pfhip_ens_req *const *rq, int n, pfhip_ens_res
   if (!d) return PFHIP_ERR_HIP;
   const EnsVec *dT = (const EnsVec *)d;
   const int *dS = (const int *)(d + bT);
-  hipLaunchKernelGGL(k_ens_vec, dim3(blk), dim3(EVB), 0, STREAM(stream), dT, dS, n,
-                     (const double *)(d + bT + bS), (const double *const *)(d + bT + bS + bC),
-                     part);
+  hipLaunchKernelGGL(k_ens_vec, dim3(blk), dim3(EVB), 0, STREAM(stream), dT,
+                     (const int2 *)(d + bT + bS), (const double *)(d + bT + bS + bB),
+                     (const double *const *)(d + bT + bS + bB + bC), part);
   LAUNCHCHK();
   if (give) {
     hipLaunchKernelGGL(k_ens_vec_final, dim3(n), dim3(EVB), 0, STREAM(stream), dT, dS,

@@ -168,3 +168,33 @@ def test_multigrid_block_launches_bitwise(gpu, shape, precision, sweeps, monkeyp
         out[blocks] = [mg.apply(b) for b in bs]
     for a, b in zip(out["0"], out["300000"]):
         assert np.array_equal(prob.interior(a), prob.interior(b))
+
+
+def test_ensemble_vector_blocks(gpu):
+    """Members whose cells a block of the ensemble's vector kernel steps
+    through differently (rows longer than a block, single rows, a remainder of
+    one cell, several blocks) against the same members advanced alone, at the
+    tolerances and the bar of the 512-member comparison."""
+    import dataclasses
+    from parflow_amd.decks import c4_member
+    api = _api()
+    members = []
+    for m, (nx, ny, nz) in enumerate([(300, 3, 20), (5, 41, 5), (3, 1, 24), (37, 28, 25)]):
+        prob, opts, _, dt = c4_member(m)
+        prob = dataclasses.replace(prob, nx=nx, ny=ny, nz=nz)
+        opts = dataclasses.replace(opts, residual_tol=1e-12, step_tol=1e-30)
+        p0 = prob.zeros()
+        z = prob.z0 + (np.arange(nz) + 0.5) * prob.dz
+        p0[1:-1, 1:-1, 1:-1] = (0.5 * nz * prob.dz - z)[:, None, None]
+        members.append((prob, opts, p0, dt))
+    ens = api.GPUEnsemble([(p, o) for p, o, _, _ in members])
+    dps = [ens.problems[i].vec(m[2]) for i, m in enumerate(members)]
+    dss = [ens.problems[i].vec() for i in range(len(members))]
+    lg = ens.advance_device(dps, dss, 0.0, [m[3] for m in members], 2)
+    assert np.all(lg["steps"] == 2)
+    for i, (prob, _, p0, dt) in enumerate(members):
+        pg, sg, l1 = ens.solvers[i].advance(p0, 0.0, dt, 2, history=False)
+        got, want = prob.interior(ens.problems[i].get(dps[i])), prob.interior(pg)
+        e = np.max(np.abs(got - want) / np.maximum(np.abs(want), 1e-3))
+        assert e < 1e-10, (i, e)
+        assert np.all(np.abs(lg["newton"][i] - l1["newton"]) <= 1), i
