@@ -198,3 +198,36 @@ def test_ensemble_vector_blocks(gpu):
         e = np.max(np.abs(got - want) / np.maximum(np.abs(want), 1e-3))
         assert e < 1e-10, (i, e)
         assert np.all(np.abs(lg["newton"][i] - l1["newton"]) <= 1), i
+
+
+@pytest.mark.parametrize("sweeps", [(1, 1), (2, 1), (0, 1), (1, 0)])
+def test_ensemble_phase_conversions(gpu, sweeps, monkeypatch):
+    """The ensemble's phase launches with the FP64 vectors converted by level
+    0's first and last half-sweep, or by passes of their own where there is no
+    such half-sweep, against every level inside one workgroup: the same bits.
+    Odd extents, so the last pair of a row has one point."""
+    import dataclasses
+    from parflow_amd.decks import c4_member
+    api = _api()
+    members = []
+    for m, (nx, ny, nz) in enumerate([(33, 20, 25), (45, 31, 30), (8, 9, 24)]):
+        prob, opts, _, dt = c4_member(m)
+        prob = dataclasses.replace(prob, nx=nx, ny=ny, nz=nz)
+        opts = dataclasses.replace(opts, num_pre_relax=sweeps[0], num_post_relax=sweeps[1])
+        p0 = prob.zeros()
+        z = prob.z0 + (np.arange(nz) + 0.5) * prob.dz
+        p0[1:-1, 1:-1, 1:-1] = (0.5 * nz * prob.dz - z)[:, None, None]
+        members.append((prob, opts, p0, dt))
+    out = []
+    for small in (None, "100000000"):
+        if small:
+            monkeypatch.setenv("PFHIP_ENS_MG_SMALL", small)
+        ens = api.GPUEnsemble([(p, o) for p, o, _, _ in members])
+        dps = [ens.problems[i].vec(m[2]) for i, m in enumerate(members)]
+        dss = [ens.problems[i].vec() for i in range(len(members))]
+        lg = ens.advance_device(dps, dss, 0.0, [m[3] for m in members], 1)
+        assert np.all(lg["steps"] == 1)
+        out.append(([ens.problems[i].get(d) for i, d in enumerate(dps)], lg))
+    for a, b in zip(out[0][0], out[1][0]):
+        assert np.array_equal(a, b)
+    assert np.array_equal(out[0][1]["gmres"], out[1][1]["gmres"])
