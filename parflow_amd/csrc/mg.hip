@@ -3122,10 +3122,10 @@ extern "C" int pfhip_mg_apply_dq(pfhip_mg *mg, const double *b, double bscale, d
 }
 
 // ---- ensemble multigrid ---------------------------------------------------------
-// The levels of a member with at most ens_small() points (the bottom of its
-// hierarchy; the whole hierarchy for small members) run inside one
-// workgroup per member, one launch for every member with a request.  The
-// larger levels of the larger members run as grid-level phases: one launch
+// The bottom of a member's hierarchy (all of it for small members) runs inside
+// one workgroup per member, one launch for every member with a request: the
+// levels that fit LDS together, or where none does those of at most ens_small()
+// points, in global memory.  The larger levels of the larger members run as grid-level phases: one launch
 // per phase and level covers that level's points of every member that has
 // it (a half-sweep, the level residual with its restriction, the prolongation,
 // the coarse operators), so no single member's one-workgroup V-cycle sets
@@ -3165,12 +3165,13 @@ struct pfhip_ens_mgplan {
   int nblk[MAXL][PS_N];
   EnsLSeg *dseg[MAXL][PS_N];          // device tables: a phase's workgroups
   void *dM;                           // device member table EnsLv<T>[n], refilled per round
-  int *dlist;                         // 0 .. n-1 (the one-workgroup kernels' members)
+  int *dlist;                         // members with their bottom in LDS, then the others
+  int nlds;                           // how many of them have it in LDS
   int use_graph;                      // replay captured launch sequences
   hipStream_t cs;                     // capture stream
   hipGraphExec_t gx[2];               // [0] coarse operators, [1] V-cycle
   long glaunch[2];                    // kernels in each captured sequence
-  long lds_bytes;                     // > 0: the one-workgroup part runs in LDS
+  long lds_bytes;                     // LDS of the largest bottom that runs there
   long launches;                      // kernel launches made so far
 };
 
@@ -3289,8 +3290,8 @@ __global__ __launch_bounds__(CWG) void k_ens_vcycle(const EnsLv<T> *__restrict__
   if (mm.lc == 0) FOR_POINTS(L0.g, mm.xout[LIDX(L0.g, i, j, k)] = (double)L0.x[LIDX(L0.g, i, j, k)]);
 }
 
-// the same with the member's levels lc .. L-1 in LDS (every member's
-// bottom fits the plan's LDS budget)
+// the same with the member's levels lc .. L-1 in LDS, for the members whose
+// plan entry says that they fit (pfhip_ens_mg_plan_create)
 template <typename T>
 __global__ __launch_bounds__(CWG) void k_ens_vcycle_lds(const EnsLv<T> *__restrict__ M,
                                                         const int *__restrict__ list)
@@ -3360,9 +3361,10 @@ extern "C" int pfhip_ens_mg_plan_create(pfhip_mg *const *mgs, int n, pfhip_ens_m
 {
   pfhip_ens_mgplan *p = (pfhip_ens_mgplan *)calloc(1, sizeof(pfhip_ens_mgplan));
   int *order = (int *)malloc(sizeof(int) * (size_t)n);
+  char *fits = (char *)calloc((size_t)n, 1);
   if (p) p->lc = (int *)malloc(sizeof(int) * (size_t)n);
-  if (!p || !order || !p->lc) {
-    free(order); pfhip_ens_mg_plan_destroy(p);
+  if (!p || !order || !fits || !p->lc) {
+    free(order); free(fits); pfhip_ens_mg_plan_destroy(p);
     pfhip_set_error("out of host memory");
     return PFHIP_ERR_NOMEM;
   }
@@ -3373,8 +3375,11 @@ extern "C" int pfhip_ens_mg_plan_create(pfhip_mg *const *mgs, int n, pfhip_ens_m
   p->use_graph = (ge && *ge) ? atoi(ge) : 1;
   int rc = PFHIP_OK;
   const long small = ens_small();
-  // the one-workgroup part in LDS: each member's first level from which
-  // every coarser level fits the budget (no PFHIP_ENS_MG_SMALL given)
+  // the one-workgroup part in LDS (no PFHIP_ENS_MG_SMALL given): a member's
+  // first level from which every coarser level fits the budget and that has
+  // at most a pair of points per thread.  A member without such a level (a
+  // hierarchy cut off by its maximum of levels) keeps its bottom in global
+  // memory, from the first level of at most ens_small() points on.
   const char *se = getenv("PFHIP_ENS_MG_SMALL");
   const char *fl = getenv("PFHIP_MG_LDS");
   const long lds_budget = (fl && *fl) ? atol(fl) : MG_LDS_DEFAULT;
@@ -3394,24 +3399,21 @@ extern "C" int pfhip_ens_mg_plan_create(pfhip_mg *const *mgs, int n, pfhip_ens_m
       rc = PFHIP_ERR_ARG;
     }
     int lc = mg->L - 1;
-    if (lds) {
-      for (int l = 0; l < mg->L; l++) {
-        const long b = lds_bottom_bytes(mg->n, l, mg->L, es);
-        if (b <= lds_budget && lds_pairs(mg->n[l]) <= CWG) {
-          lc = l;
-          if (b > p->lds_bytes) p->lds_bytes = b;
-          break;
-        }
-      }
-    } else {
-      for (int l = 0; l < mg->L; l++)
-        if (npts(mg->n[l]) <= small) { lc = l; break; }
+    for (int l = 0; lds && l < mg->L && !fits[m]; l++) {
+      const long b = lds_bottom_bytes(mg->n, l, mg->L, es);
+      if (b > lds_budget || lds_pairs(mg->n[l]) > CWG) continue;
+      lc = l;
+      fits[m] = 1;
+      p->nlds++;
+      if (b > p->lds_bytes) p->lds_bytes = b;
     }
+    for (int l = 0; l < mg->L && !fits[m]; l++)
+      if (npts(mg->n[l]) <= small) { lc = l; break; }
     p->lc[m] = lc;
     if (lc > p->G) p->G = lc;
     order[m] = m;
   }
-  if (rc == PFHIP_OK && p->lds_bytes > 0) {
+  if (rc == PFHIP_OK && p->nlds > 0) {
     hipError_t e = (p->prec == 64)
         ? hipFuncSetAttribute((const void *)k_ens_vcycle_lds<double>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)p->lds_bytes)
@@ -3458,7 +3460,7 @@ extern "C" int pfhip_ens_mg_plan_create(pfhip_mg *const *mgs, int n, pfhip_ens_m
   if (rc == PFHIP_OK) rc = pfhip_malloc(&p->dM, (long)mb);
   if (rc == PFHIP_OK) rc = pfhip_malloc((void **)&p->dlist, (long)sizeof(int) * n);
   if (rc == PFHIP_OK) {
-    for (int m = 0; m < n; m++) order[m] = m;
+    for (int m = 0, a = 0, b = p->nlds; m < n; m++) order[fits[m] ? a++ : b++] = m;
     if (hipMemcpy(p->dlist, order, sizeof(int) * n, hipMemcpyHostToDevice) != hipSuccess) {
       pfhip_set_error("hipMemcpy of the ensemble member list");
       rc = PFHIP_ERR_HIP;
@@ -3470,6 +3472,7 @@ extern "C" int pfhip_ens_mg_plan_create(pfhip_mg *const *mgs, int n, pfhip_ens_m
     rc = PFHIP_ERR_HIP;
   }
   free(order);
+  free(fits);
   if (rc) { pfhip_ens_mg_plan_destroy(p); return rc; }
   *out = p;
   return PFHIP_OK;
@@ -3527,13 +3530,18 @@ static int ens_sequence(pfhip_ens_mgplan *p, int apply, hipStream_t s)
     ens_phase<T>(p, l, PS_COARSE, EL_RESTRICT, 0, 0, 0, s);
     LAUNCHCHK();
   }
-  if (p->lds_bytes > 0)
-    hipLaunchKernelGGL(k_ens_vcycle_lds<T>, dim3(p->n), dim3(CWG), (unsigned)p->lds_bytes, s,
+  if (p->nlds > 0) {
+    hipLaunchKernelGGL(k_ens_vcycle_lds<T>, dim3(p->nlds), dim3(CWG), (unsigned)p->lds_bytes, s,
                        dM, p->dlist);
-  else
-    hipLaunchKernelGGL(k_ens_vcycle<T>, dim3(p->n), dim3(CWG), 0, s, dM, p->dlist);
-  LAUNCHCHK();
-  p->launches++;
+    LAUNCHCHK();
+    p->launches++;
+  }
+  if (p->n > p->nlds) {
+    hipLaunchKernelGGL(k_ens_vcycle<T>, dim3(p->n - p->nlds), dim3(CWG), 0, s, dM,
+                       p->dlist + p->nlds);
+    LAUNCHCHK();
+    p->launches++;
+  }
   for (int l = p->G - 1; l >= 0; l--) {
     ens_phase<T>(p, l, PS_FINE, EL_PROLONG, 0, 0, 0, s);
     ens_sweeps<T>(p, l, 0, p->post, l == 0 ? EC_OUT : EC_NONE, s);

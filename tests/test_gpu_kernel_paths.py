@@ -231,3 +231,43 @@ def test_ensemble_phase_conversions(gpu, sweeps, monkeypatch):
     for a, b in zip(out[0][0], out[1][0]):
         assert np.array_equal(a, b)
     assert np.array_equal(out[0][1]["gmres"], out[1][1]["gmres"])
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_ensemble_bottoms_that_do_not_fit_lds(gpu, precision, monkeypatch):
+    """Members whose hierarchies are cut off at a level that the LDS bottom
+    cannot take (1500 pairs of points; 12,000 points) beside one that it
+    takes: the same bits as with every level in one workgroup in global
+    memory, and the members' own solutions (at the deck's tolerances the two
+    paths differ by up to 5e-8)."""
+    import dataclasses
+    from parflow_amd.decks import c4_member
+    api = _api()
+    members = []
+    for m, (nx, ny, nz, levels) in enumerate([(12, 10, 20, 100), (30, 20, 20, 3), (40, 30, 20, 2),
+                                              (9, 30, 21, 100)]):
+        prob, opts, _, dt = c4_member(m)
+        prob = dataclasses.replace(prob, nx=nx, ny=ny, nz=nz)
+        opts = dataclasses.replace(opts, max_levels=levels)
+        p0 = prob.zeros()
+        z = prob.z0 + (np.arange(nz) + 0.5) * prob.dz
+        p0[1:-1, 1:-1, 1:-1] = (0.5 * nz * prob.dz - z)[:, None, None]
+        members.append((prob, opts, p0, dt))
+    out = []
+    for small in (None, "100000000"):
+        if small:
+            monkeypatch.setenv("PFHIP_ENS_MG_SMALL", small)
+        ens = api.GPUEnsemble([(p, o) for p, o, _, _ in members], precision=precision)
+        dps = [ens.problems[i].vec(m[2]) for i, m in enumerate(members)]
+        dss = [ens.problems[i].vec() for i in range(len(members))]
+        lg = ens.advance_device(dps, dss, 0.0, [m[3] for m in members], 2)
+        assert np.all(lg["steps"] == 2)
+        out.append(([ens.problems[i].get(d) for i, d in enumerate(dps)], lg))
+    for a, b in zip(out[0][0], out[1][0]):
+        assert np.array_equal(a, b)
+    assert np.array_equal(out[0][1]["gmres"], out[1][1]["gmres"])
+    for i, (prob, _, p0, dt) in enumerate(members):
+        pg, _, l1 = ens.solvers[i].advance(p0, 0.0, dt, 2, history=False)
+        got, want = prob.interior(out[0][0][i]), prob.interior(pg)
+        assert np.max(np.abs(got - want) / np.maximum(np.abs(want), 1e-3)) < 1e-6, i
+        assert np.all(np.abs(out[0][1]["newton"][i] - l1["newton"]) <= 1), i
