@@ -2619,8 +2619,8 @@ extern "C" int pfhip_nl_function_eval(pfhip_problem *pb, const double *p, double
 // marches 16 planes: kr*rho of every cell is evaluated once, in place (the
 // tile's west and south neighbours again), the lateral neighbours come from
 // LDS and the lower one from a register.  HBM bounds it: p, alpha, n and K
-// read (32 B isotropic), three velocities written (24 B).  512x512x32: 104 us
-// + 15 us for the domain's faces, 4.5 TB/s (64 x 4 tiles 113 us, 64 x 16
+// read (32 B isotropic), three velocities written (24 B).  512x512x32: 106 us
+// + 15 us for the domain's faces, 4.4 TB/s (64 x 4 tiles 113 us, 64 x 16
 // 110 us, 32 planes 108 us); a closure pass that stored kr*rho and a pass
 // over the faces took 51 + 139 us.
 // --------------------------------------------------------------------------
@@ -2659,30 +2659,41 @@ __device__ __forceinline__ double bc_face_velocity(const ResArgs &A, int fc, int
 
 #define FVY 8
 #define FVZ 16
-// a / b for a constant b with rb = 1 / b rounded to nearest: the quotient
+// a / b for a constant b > 0 with rb = 1 / b rounded to nearest: the quotient
 // corrected once by its exact remainder, which rounds it as the division does
-// (Markstein, IBM J. Res. Dev. 34 (1990)), in three instructions
+// (Markstein, IBM J. Res. Dev. 34 (1990)), in three instructions and one for
+// the sign of a zero.  An infinite a or an overflow gives NaN or infinity, and
+// below the normal range the last bit may differ.
 __device__ __forceinline__ double div_const(double a, double b, double rb)
 {
   const double q = a * rb;
-  return fma(fma(-b, q, a), rb, q);
+  return copysign(fma(fma(-b, q, a), rb, q), a);
 }
-// flux_xy and flux_z over the face area ff: the same operands and order
+// flux_xy and flux_z over the face area ff with reciprocals for the quotients:
+// the same values where size, which they add to, stays below VEL_LIMIT.  It
+// holds their numerator over mu and ff, which an infinite or overflowing
+// operand, product or quotient before it leaves infinite or NaN, and the sum of
+// the permeabilities, scaled to pass the limit from 2^1000 on, where its
+// reciprocal nears the end of the normal range.
+#define VEL_LIMIT 0x1p400
+__device__ __forceinline__ bool vel_const_ok(double c) { return c > 0x1p-200 && c < 0x1p200; }
 __device__ __forceinline__ double vel_xy(double pa, double pb, double ka, double kb, double kra,
                                          double krb, double ff, double iff, double d, double id,
-                                         double gc, double mu, double imu)
+                                         double gc, double mu, double imu, double &size)
 {
   const double dd = div_const(pa - pb, d, id);
-  return div_const(div_const(ff * hmean_f(ka, kb) * dd * gc * upw(dd * gc, 0.0, kra, krb), mu,
-                             imu), ff, iff);
+  const double num = ff * hmean_f(ka, kb) * dd * gc * upw(dd * gc, 0.0, kra, krb);
+  size += fma(fabs(ka + kb), 0x1p-600, fabs(num));
+  return div_const(div_const(num, mu, imu), ff, iff);
 }
 __device__ __forceinline__ double vel_z(double pa, double pb, double ka, double kb, double kra,
                                         double krb, double ff, double iff, double dz, double idz,
-                                        double hrg, double mu, double imu)
+                                        double hrg, double mu, double imu, double &size)
 {
   const double lc = div_const(pa, dz, idz) - hrg, uc = div_const(pb, dz, idz) + hrg;
-  return div_const(div_const(ff * hmean_f(ka, kb) * (lc - uc) * upw(lc, uc, kra, krb), mu, imu),
-                   ff, iff);
+  const double num = ff * hmean_f(ka, kb) * (lc - uc) * upw(lc, uc, kra, krb);
+  size += fma(fabs(ka + kb), 0x1p-600, fabs(num));
+  return div_const(div_const(num, mu, imu), ff, iff);
 }
 // a cell's inputs on one plane
 struct VelIn { double p, al, n, kx, ky, kz; };
@@ -2709,6 +2720,11 @@ __global__ __launch_bounds__(64 * FVY) void k_face_velocity(ResArgs A, VelOut V)
   const double ffx = dy * dz, ffy = dx * dz, ffz = dx * dy;
   const double iffx = 1.0 / ffx, iffy = 1.0 / ffy, iffz = 1.0 / ffz;
   const double hrg = 0.5 * rho * grav * 1.0;
+  // numerators from here on are divided in full, all of them where a divisor
+  // is out of proportion
+  const bool ok = vel_const_ok(ffx) && vel_const_ok(ffy) && vel_const_ok(ffz) &&
+                  vel_const_ok(dx) && vel_const_ok(dy) && vel_const_ok(dz) && vel_const_ok(mu);
+  const double lim = ok ? VEL_LIMIT : 0.0;
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   int bx, by, bz;
   tile_of_block(bx, by, bz);
@@ -2728,6 +2744,13 @@ __global__ __launch_bounds__(64 * FVY) void k_face_velocity(ResArgs A, VelOut V)
   const int hcol = halo ? (bx * 64 + hx) + (by * FVY + hy) * g.sy : col;
   const int hls = hy * W + hx;
   const int k0 = bz * FVZ, k1 = min(k0 + FVZ, g.nz);
+  // zeros where there is no neighbour
+  if (tid < FVY + 64 && !halo) {
+    for (int q = 0; q < 2; q++) {
+      s_p[q][hls] = s_kr[q][hls] = s_k[q][hls] = 0.0;
+      if constexpr (!ISO) s_ky[q][hls] = 0.0;
+    }
+  }
   double p_m = 0.0, kr_m = 0.0, kz_m = 0.0;
   if (k0 > 0) {
     VelIn m;
@@ -2764,14 +2787,23 @@ __global__ __launch_bounds__(64 * FVY) void k_face_velocity(ResArgs A, VelOut V)
       const long oy = i + (long)g.nx * (j + (long)(g.ny + 1) * k);
       const long oz = i + (long)g.nx * (j + (long)g.ny * k);
       const int w = ls - 1, sth = ls - W;
-      if (i > 0)
-        V.vx[ox] = vel_xy(s_p[q][w], c.p, s_k[q][w], c.kx, s_kr[q][w], kr, ffx, iffx, dx, A.idx,
-                          grav, mu, A.imu);
-      if (j > 0)
-        V.vy[oy] = vel_xy(s_p[q][sth], c.p, ky_s[sth], c.ky, s_kr[q][sth], kr, ffy, iffy, dy,
-                          A.idy, grav, mu, A.imu);
-      if (k > 0)
-        V.vz[oz] = vel_z(p_m, c.p, kz_m, c.kz, kr_m, kr, ffz, iffz, dz, A.idz, hrg, mu, A.imu);
+      double size = 0.0;
+      double ux = vel_xy(s_p[q][w], c.p, s_k[q][w], c.kx, s_kr[q][w], kr, ffx, iffx, dx, A.idx,
+                         grav, mu, A.imu, size);
+      double uy = vel_xy(s_p[q][sth], c.p, ky_s[sth], c.ky, s_kr[q][sth], kr, ffy, iffy, dy,
+                         A.idy, grav, mu, A.imu, size);
+      double uz = vel_z(p_m, c.p, kz_m, c.kz, kr_m, kr, ffz, iffz, dz, A.idz, hrg, mu, A.imu,
+                        size);
+      // one test for the three (NaN fails it): 106 us at 512x512x32, 103
+      // without it; 109 with a test a face, 115 with plain divisions
+      if (!(size < lim)) {
+        ux = flux_xy(s_p[q][w], c.p, s_k[q][w], c.kx, s_kr[q][w], kr, ffx, dx, grav, mu) / ffx;
+        uy = flux_xy(s_p[q][sth], c.p, ky_s[sth], c.ky, s_kr[q][sth], kr, ffy, dy, grav, mu) / ffy;
+        uz = flux_z(p_m, c.p, kz_m, c.kz, kr_m, kr, ffz, dz, rho, grav, mu) / ffz;
+      }
+      if (i > 0) V.vx[ox] = ux;
+      if (j > 0) V.vy[oy] = uy;
+      if (k > 0) V.vz[oz] = uz;
     }
     p_m = c.p; kr_m = kr; kz_m = c.kz;
   }

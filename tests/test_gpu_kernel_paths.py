@@ -69,6 +69,54 @@ def test_face_velocity_tiles(gpu, shape, overland, dirs):
         assert np.max(np.abs(a - b)) <= 1e-12 * scale
 
 
+@pytest.mark.parametrize("iso", [True, False])
+def test_face_velocity_infinities_and_zeros(gpu, iso):
+    """Interior face velocities of saturated cells (kr = 1) with infinite and
+    overflowing pressures, differences and permeabilities and with zero ones:
+    NaN, the infinities and the sign of a zero as the oracle's divisions leave
+    them, finite values to the rounding of their dozen operations (z faces:
+    of the two heads they subtract)."""
+    import dataclasses
+    api = _api()
+    prob = cases.hetero(70, 17, 20, seed=41)
+    rng = np.random.default_rng(42)
+    K = []
+    for q in range(1 if iso else 3):
+        k = np.exp(rng.normal(np.log(0.1), 1.0, (prob.nz, prob.ny, prob.nx)))
+        k.ravel()[rng.choice(k.size, 900, replace=False)] = np.resize(
+            [0.0, 1e200, 1.7e308, np.inf, 1e-200], 900)
+        K.append(k)
+    prob = dataclasses.replace(prob, kx=K[0], ky=K[-1] if iso else K[1], kz=K[-1])
+    p = prob.zeros()
+    inner = rng.uniform(0.0, 50.0, (prob.nz, prob.ny, prob.nx))
+    inner.ravel()[rng.choice(inner.size, 1500, replace=False)] = np.resize(
+        [np.inf, 1.7e308, 0.0, -0.0, 1e-310, 1e160], 1500)
+    p[1:-1, 1:-1, 1:-1] = inner
+    got = api.GPUProblem(prob).face_velocity(p, p, 0.1, 0.1)
+    want = O.face_velocity(O.OracleProblem(prob), p, p, 0.1, 0.1)
+    seen = np.zeros(3, dtype=int)
+    for ax, (a, b) in enumerate(zip(got, want)):
+        face = [slice(None)] * 3
+        face[2 - ax] = slice(1, -1)
+        a, b = a[tuple(face)], b[tuple(face)]
+        assert np.array_equal(np.isnan(a), np.isnan(b))
+        assert np.array_equal(np.isinf(a), np.isinf(b))
+        signed = np.isinf(b) | (b == 0)
+        assert np.array_equal(np.signbit(a[signed]), np.signbit(b[signed]))
+        assert np.all(a[b == 0] == 0)
+        fin = np.isfinite(b) & (b != 0)
+        with np.errstate(all="ignore"):
+            if ax < 2:
+                bar = 4e-15 * np.abs(b)
+            else:
+                k = K[-1]
+                h = 2 * k[:-1] * k[1:] / (k[:-1] + k[1:])
+                bar = 4e-15 * h * (inner[:-1] / prob.dz + inner[1:] / prob.dz + 1)
+            assert np.all(np.abs(a - b)[fin] <= np.maximum(bar, 1e-300)[fin])
+        seen += [np.sum(np.isnan(b)), np.sum(np.isinf(b)), np.sum((b == 0) & np.signbit(b))]
+    assert np.all(seen > 0)
+
+
 @pytest.mark.parametrize("shape", [(1, 1, 1), (2, 2, 2), (70, 9, 5)])
 @pytest.mark.parametrize("with_src", [False, True])
 def test_water_balance_fluxes_shell(gpu, shape, with_src):
