@@ -55,6 +55,14 @@ extern "C" const char *pfhip_last_error(void) { return g_err; }
 
 #define STREAM(s) ((hipStream_t)(s))
 
+// pinned memory that a kernel writes while the host polls it, or reads while
+// the host fills it for the next one: coherent as asked for, not as the
+// runtime's default has it
+static hipError_t pinned_shared(void **p, size_t bytes)
+{
+  return hipHostMalloc(p, bytes, hipHostMallocCoherent);
+}
+
 // --------------------------------------------------------------------------
 // live timing with HIP events (pfhip_prof_*): when a timer id is enabled,
 // every launch of that kernel (or every call of that solver phase) is
@@ -388,7 +396,7 @@ extern "C" int pfhip_problem_create(const pfhip_problem_desc *desc,
   }
   if (rc == PFHIP_OK) {
     // the results and, behind them, the sequence number of the last ones
-    hipError_t e = hipHostMalloc((void **)&pb->h_red, sizeof(double) * (PFHIP_RED_SLOTS + 1));
+    hipError_t e = pinned_shared((void **)&pb->h_red, sizeof(double) * (PFHIP_RED_SLOTS + 1));
     if (e != hipSuccess) { pfhip_set_error("hipHostMalloc"); rc = PFHIP_ERR_NOMEM; }
     else memset(pb->h_red, 0, sizeof(double) * (PFHIP_RED_SLOTS + 1));
   }
@@ -4059,7 +4067,7 @@ extern "C" int pfhip_ens_results_create(pfhip_ens_results *r, long n)
   r->host = nullptr;
   r->ticket = nullptr;
   r->seq = 0;
-  HIPCHK(hipHostMalloc((void **)&r->host, sizeof(double) * (n + 1), hipHostMallocDefault));
+  HIPCHK(pinned_shared((void **)&r->host, sizeof(double) * (n + 1)));
   r->flag = (unsigned long long *)(r->host + n);
   *r->flag = 0;
   HIPCHK(hipMalloc((void **)&r->ticket, sizeof(unsigned)));
@@ -4481,7 +4489,7 @@ extern "C" int pfhip_ens_stage_create(pfhip_ens_stage *st, long cap)
   st->cap = cap;
   st->host = nullptr;
   st->dev = nullptr;
-  HIPCHK(hipHostMalloc((void **)&st->host, cap, hipHostMallocDefault));
+  HIPCHK(pinned_shared((void **)&st->host, (size_t)cap));
   HIPCHK(hipMalloc((void **)&st->dev, cap));
   return PFHIP_OK;
 }

@@ -52,6 +52,29 @@ def test_reduction_results_reach_the_host(gpu, shape):
             assert abs(b.value - np.max(np.abs(Y) / (1 + np.abs(X)))) <= 1e-15 * b.value
 
 
+def test_shared_pinned_memory_is_coherent(gpu):
+    """The ensemble's result slots and staging ring, which kernels and the host
+    use without a copy or a synchronisation between them, are allocated
+    coherent, whatever the runtime's default is."""
+    class Results(C.Structure):
+        _fields_ = [("host", C.c_void_p), ("flag", C.c_void_p), ("seq", C.c_ulonglong),
+                    ("ticket", C.c_void_p)]
+
+    class Stage(C.Structure):
+        _fields_ = [("host", C.c_void_p), ("dev", C.c_void_p), ("off", C.c_long),
+                    ("cap", C.c_long)]
+    api = _api()
+    lib = api.lib()                    # and the HIP runtime it is linked to
+    r, st, flags = Results(), Stage(), C.c_uint()
+    api.check(lib.pfhip_ens_results_create(C.byref(r), C.c_long(64)), "results")
+    api.check(lib.pfhip_ens_stage_create(C.byref(st), C.c_long(1 << 16)), "stage")
+    for p in (r.host, st.host):
+        assert lib.hipHostGetFlags(C.byref(flags), C.c_void_p(p)) == 0
+        assert flags.value & 0x40000000          # hipHostMallocCoherent
+    lib.pfhip_ens_results_destroy(C.byref(r))
+    lib.pfhip_ens_stage_destroy(C.byref(st))
+
+
 @pytest.mark.parametrize("shape", [(1, 1, 1), (64, 8, 16), (65, 9, 17), (130, 3, 33)])
 @pytest.mark.parametrize("overland,dirs", [(False, True), (True, False)])
 def test_face_velocity_tiles(gpu, shape, overland, dirs):
