@@ -2,6 +2,7 @@
 can go wrong: tile edges, remainders, the smallest grids.  Bars are the
 rounding of the summed terms, as in the parity tests."""
 import ctypes as C
+import dataclasses
 
 import numpy as np
 import pytest
@@ -21,6 +22,19 @@ def _field(prob, rng, ghost=1e9):
     a = np.full(prob.shape, ghost)
     a[1:-1, 1:-1, 1:-1] = rng.normal(size=(prob.nz, prob.ny, prob.nx))
     return a
+
+
+def _form(prob, form):
+    """prob with independent kx, ky and kz ("aniso"), or with uniform van
+    Genuchten parameters and kr from a table ("table")."""
+    if form == "aniso":
+        rng = np.random.default_rng(51)
+        ky, kz = (np.exp(rng.normal(np.log(0.1), 1.0, (prob.nz, prob.ny, prob.nx)))
+                  for _ in range(2))
+        return dataclasses.replace(prob, ky=ky, kz=kz)
+    if form == "table":
+        return dataclasses.replace(prob, alpha=1.3, nvg=2.3, vg_table=(40, -6.0, "Spline"))
+    return prob
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 2), (5, 3, 2), (65, 33, 40)])
@@ -77,11 +91,13 @@ def test_shared_pinned_memory_is_coherent(gpu):
 
 @pytest.mark.parametrize("shape", [(1, 1, 1), (64, 8, 16), (65, 9, 17), (130, 3, 33)])
 @pytest.mark.parametrize("overland,dirs", [(False, True), (True, False)])
-def test_face_velocity_tiles(gpu, shape, overland, dirs):
+@pytest.mark.parametrize("form", ["iso", "aniso", "table"])
+def test_face_velocity_tiles(gpu, shape, overland, dirs, form):
     """Face velocities over grids that fill, exceed and fall short of the
-    kernel's 64 x 8 x 16 tiles, against the oracle."""
+    kernel's 64 x 8 x 16 tiles, with one permeability, three, and kr from a
+    lookup table, against the oracle."""
     api = _api()
-    prob = cases.hetero(*shape, seed=4, overland=overland, dir_sides=dirs)
+    prob = _form(cases.hetero(*shape, seed=4, overland=overland, dir_sides=dirs), form)
     gp, op = api.GPUProblem(prob), O.OracleProblem(prob)
     p, p_old = cases.random_pressure(prob, seed=5), cases.random_pressure(prob, seed=6)
     t = 0.1
@@ -99,7 +115,6 @@ def test_face_velocity_infinities_and_zeros(gpu, iso):
     NaN, the infinities and the sign of a zero as the oracle's divisions leave
     them, finite values to the rounding of their dozen operations (z faces:
     of the two heads they subtract)."""
-    import dataclasses
     api = _api()
     prob = cases.hetero(70, 17, 20, seed=41)
     rng = np.random.default_rng(42)
@@ -167,12 +182,17 @@ def test_water_balance_fluxes_shell(gpu, shape, with_src):
         assert f[3] == 0.0
 
 
-@pytest.mark.parametrize("shape", [(1, 1, 1), (64, 8, 2), (65, 9, 3), (200, 130, 9), (513, 130, 35)])
-def test_residual_and_jacobian_plane_chunks(gpu, shape):
-    """F and both Jacobians where the tiles march 2, 4 and 8 planes and the
-    last chunk is cut short, against the oracle."""
+@pytest.mark.parametrize("shape,form", [
+    ((1, 1, 1), "iso"), ((64, 8, 2), "iso"), ((65, 9, 3), "iso"), ((200, 130, 9), "iso"),
+    ((513, 130, 13), "iso"), ((513, 130, 35), "iso"), ((513, 262, 18), "iso"),
+    ((65, 9, 3), "aniso"), ((130, 20, 37), "aniso"), ((513, 130, 13), "aniso"),
+    ((65, 9, 5), "table")])
+def test_residual_and_jacobian_plane_chunks(gpu, shape, form):
+    """F and both Jacobians where the tiles march 2 planes (grids below 513 x
+    130), 4, 8 and 16 (513 x 130 x 13 and 35, 513 x 262 x 18) and the last
+    chunk is cut short, against the oracle."""
     api = _api()
-    prob = cases.hetero(*shape, seed=11, dir_sides=True)
+    prob = _form(cases.hetero(*shape, seed=11, dir_sides=True), form)
     gp, op = api.GPUProblem(prob), O.OracleProblem(prob)
     p, p_old = cases.random_pressure(prob, seed=12), cases.random_pressure(prob, seed=13)
     s_old = O.saturation(op, p_old, 0)
@@ -246,7 +266,6 @@ def test_ensemble_vector_blocks(gpu):
     through differently (rows longer than a block, single rows, a remainder of
     one cell, several blocks) against the same members advanced alone, at the
     tolerances and the bar of the 512-member comparison."""
-    import dataclasses
     from parflow_amd.decks import c4_member
     api = _api()
     members = []
@@ -277,7 +296,6 @@ def test_ensemble_phase_conversions(gpu, sweeps, monkeypatch):
     0's first and last half-sweep, or by passes of their own where there is no
     such half-sweep, against every level inside one workgroup: the same bits.
     Odd extents, so the last pair of a row has one point."""
-    import dataclasses
     from parflow_amd.decks import c4_member
     api = _api()
     members = []
@@ -311,7 +329,6 @@ def test_ensemble_bottoms_that_do_not_fit_lds(gpu, precision, monkeypatch):
     takes: the same bits as with every level in one workgroup in global
     memory, and the members' own solutions (at the deck's tolerances the two
     paths differ by up to 5e-8)."""
-    import dataclasses
     from parflow_amd.decks import c4_member
     api = _api()
     members = []

@@ -553,6 +553,14 @@ def test_multigrid_full_storage(gpu, precision, shape):
         assert _relmax(_I(prob, xg), _I(prob, xo)) < tol, (pre, post, sym)
 
 
+@pytest.fixture(params=["300000", "0"], ids=["blocks", "separate"])
+def level_launches(request, monkeypatch):
+    """The grid levels visited by one block launch each (the default at the
+    tests' sizes), and by the separate launches that larger levels take."""
+    monkeypatch.setenv("PFHIP_MG_BLOCK", request.param)
+
+
+@pytest.mark.usefixtures("level_launches")
 @pytest.mark.parametrize("shape", [(70, 40, 24), (130, 20, 18)])
 @pytest.mark.parametrize("precision", [64, 32])
 @pytest.mark.parametrize("fuse", [0, 1])
@@ -595,14 +603,14 @@ def test_multigrid_grid_levels(gpu, precision, fuse, shape, monkeypatch):
 
 
 @pytest.mark.parametrize("precision", [64, 32])
-@pytest.mark.parametrize("variant", [0, 7])
+@pytest.mark.parametrize("variant", [0, 7, ""], ids=["0", "7", "blocks"])
 def test_multigrid_graph_replay(gpu, precision, variant, monkeypatch):
     """The V-cycle replayed from its captured hipGraph against the same
     hierarchy launching directly (PFHIP_MG_GRAPH=0): six V-cycles on new
     right-hand sides, the direct hierarchy's V-cycle and a host round trip
     between the replays, every replay identical to the last bit; and the
     oracle bar.  The tile shape is forced, so both hierarchies run the same
-    kernels."""
+    kernels; without one every grid level is visited by block launches."""
     api = _api()
     monkeypatch.setenv("PFHIP_RBGS_VARIANT", str(variant))
     prob = cases.hetero(70, 40, 24, seed=41, dir_sides=True)
@@ -695,6 +703,7 @@ def test_multigrid_pair_shapes(gpu, variant, shape, precision, monkeypatch):
     assert err < (1e-11 if precision == 64 else 2e-5), err
 
 
+@pytest.mark.usefixtures("level_launches")
 @pytest.mark.parametrize("precision", [32, 64])
 def test_multigrid_fp64_vector_alignment(gpu, precision):
     """The V-cycle's first pair reads the FP64 right-hand side and its last
@@ -926,6 +935,7 @@ def test_cgs2_scaled_basis_matches_scaled_vectors(gpu, k):
     assert np.array_equal(_I(prob, gp.get(wa)), _I(prob, gp.get(wb)))
 
 
+@pytest.mark.usefixtures("level_launches")
 @pytest.mark.parametrize("precision,shape", [(32, (70, 40, 24)), (64, (70, 40, 24)),
                                              (32, (71, 30, 20))])
 def test_mg_apply_scaled_matches_scaled_vector(gpu, precision, shape, monkeypatch):
@@ -961,6 +971,7 @@ def test_mg_apply_scaled_matches_scaled_vector(gpu, precision, shape, monkeypatc
             assert np.array_equal(ia, ib), (graph, c, _relmax(ia, ib))
 
 
+@pytest.mark.usefixtures("level_launches")
 @pytest.mark.parametrize("precision,shape", [(32, (70, 40, 24)), (64, (70, 40, 24)),
                                              (32, (71, 30, 20)), (32, (128, 30, 37))])
 def test_mg_apply_dq_sums(gpu, precision, shape, monkeypatch):
