@@ -83,12 +83,12 @@ def kernel_bytes_per_cell(gp):
 
 PROF_KERNELS = (
     # (key, api prof id name, kernel as rocprofv3 names it)
-    ("residual", "PROF_RESIDUAL", "k_residual_pf<64, 8, 16, *, 0> (NlFunctionEval)"),
+    ("residual", "PROF_RESIDUAL", "k_residual_pf<64, 8, *, 0> (NlFunctionEval)"),
     ("residual_jv", "PROF_RESIDUAL_JV",
-     "k_residual_pf<64, 8, 16, *, 1> (difference-quotient J.v)"),
+     "k_residual_pf<64, 8, *, 1> (difference-quotient J.v)"),
     ("residual_step", "PROF_RESIDUAL_STEP",
-     "k_residual_pf<64, 8, 16, *, 2> (line-search trial point)"),
-    ("jacobian", "PROF_JACOBIAN", "k_jacobian_pf<64, 8, 16, *, true, float> (PC matrix)"),
+     "k_residual_pf<64, 8, *, 2> (line-search trial point)"),
+    ("jacobian", "PROF_JACOBIAN", "k_jacobian_pf<64, 8, *, true, float> (PC matrix)"),
     ("rbgs_pair", "PROF_RBGS", "k_rbgs_pair2<float, ...> FP32 operands"),
     ("rbgs_pair_dout", "PROF_RBGS_DOUT", "k_rbgs_pair2<float, ...> FP64 result"),
     ("rbgs_pair_din", "PROF_RBGS_DIN", "k_rbgs_pair2<float, ...> FP64 right-hand side"),

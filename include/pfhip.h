@@ -435,7 +435,8 @@ int  pfhip_ensemble_advance_richards(pfhip_ensemble *e, double *const *p,
                                      const double *dt, int nsteps,
                                      int max_conv_failures, int *newton, int *gmres,
                                      int *fevals, int *steps_done);
-/* scheduler rounds and batched launches of the last advance */
+/* scheduler rounds and batched launches of the last advance (the finishing
+ * launch of a vector operation and the table copies not counted) */
 int  pfhip_ensemble_stats(pfhip_ensemble *e, long *rounds, long *launches);
 
 /* ---- live kernel and phase timing (HIP events on the launching stream) */

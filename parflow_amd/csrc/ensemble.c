@@ -290,9 +290,7 @@ static int e_mg_apply(pfhip_mg *mg, const double *b, double *x, void *st)
   return submit();
 }
 
-/* Once per Newton solve: the member's own small launches/copies, enqueued
- * behind the batched work.  Its BC staging is reused only after the
- * reductions of that solve, which synchronise the stream. */
+/* Once per Newton solve; the values are staged in the ensemble's ring. */
 static int e_bc_pressure(pfhip_problem *pb, double t, void *st)
 {
   pfhip_ens_req *r = new_req(PFHIP_EOP_BC);

@@ -254,8 +254,9 @@ typedef struct pfhip_ens_req {
 } pfhip_ens_req;
 
 /* staging ring for the per-launch member tables: pinned host memory copied
- * asynchronously to its device twin; off returns to 0 after a stream
- * synchronisation */
+ * to its device twin by a kernel (large blocks by an asynchronous copy); off
+ * returns to 0 when the stream has been waited for, or when results have come
+ * back with nothing queued behind them */
 typedef struct pfhip_ens_stage {
   char *host, *dev;
   long off, cap;
