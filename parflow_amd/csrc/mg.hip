@@ -18,11 +18,14 @@
 //    renumbered so each of the 8 XCDs owns a contiguous z-range (the
 //    hardware deals workgroups to XCDs round-robin; without the renumbering
 //    the z-neighbour planes of a tile sit in other XCDs' L2);
-//  * every level with <= MG_SMALL_DEFAULT points (the bottom of the V-cycle,
-//    a dozen levels of a semicoarsened hierarchy; PFHIP_MG_SMALL overrides
-//    the bound) runs inside ONE workgroup of 1024 threads, phase by phase
-//    with __syncthreads, instead of ~100 launches that are pure launch
-//    latency.
+//  * levels of up to BLOCK_POINTS points (symmetric storage) take one launch a
+//    visit, a block of points with its rim per workgroup (k_lvl_block);
+//  * the bottom of the V-cycle, a dozen levels of a semicoarsened hierarchy,
+//    runs inside ONE workgroup of 1024 threads, phase by phase, instead of
+//    ~100 launches that are pure launch latency: in LDS the levels that fit
+//    it together and have at most a pair of points per thread; without LDS,
+//    or with full storage, those of at most MG_SMALL_DEFAULT points
+//    (PFHIP_MG_SMALL overrides the bound, and then LDS is not used).
 #include <hip/hip_runtime.h>
 #include <stdlib.h>
 #include <string.h>
